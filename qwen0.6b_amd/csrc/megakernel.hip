@@ -407,7 +407,7 @@ int launch(KParams& P, hipStream_t stream, bool fixed = false) {
 
 // prefill activations for up to MAX_SEQ_LIMIT positions: residual X fp32 [n, 1024], q and the
 // attention output fp16 [n, 2048] each, SiLU * up fp16 [n, 3072], the next RMSNorm's gained input
-// fp16 [n, 1024] and its block sums of squares fp32 [n, 32], then the barrier counters and
+// fp16 [n, 1024] and its block sums of squares fp32 [n, 64], then the barrier counters and
 // the split attention items' arrival counters (zeroed before every launch), the timestamps and
 // the split items' partial results
 constexpr long PF_X = 0;
@@ -416,16 +416,16 @@ constexpr long PF_AO = PF_Q + (long)MAX_SEQ_LIMIT * QSZ * 2;
 constexpr long PF_IM = PF_AO + (long)MAX_SEQ_LIMIT * QSZ * 2;
 constexpr long PF_XN = PF_IM + (long)MAX_SEQ_LIMIT * INTER * 2;
 constexpr long PF_SSQ = PF_XN + (long)MAX_SEQ_LIMIT * HIDDEN * 2;
-constexpr long PF_BAR = PF_SSQ + (long)MAX_SEQ_LIMIT * 32 * 4;
+constexpr long PF_BAR = PF_SSQ + (long)MAX_SEQ_LIMIT * pf::SSB * 4;
 constexpr int PF_NTS = 1 + 1 + 5 * MAX_LAYERS;  // launch start, then every grid barrier
-constexpr long PF_BAR_LINES = 4096;              // barrier words: 8 XCDs x 64 arrivals, then 8 leaders
+constexpr long PF_BAR_LINES = 4096;              // barrier words: 8 XCDs x 64 arrivals, 8 copies of 8 leaders
 constexpr long PF_ACNT = PF_BAR + PF_BAR_LINES;
 constexpr long PF_BAR_BYTES = PF_BAR_LINES + 4L * pf::MAX_QB * NKV;
 constexpr long PF_TS = PF_BAR + PF_BAR_BYTES;
 constexpr long PF_PART = (PF_TS + 8L * ((PF_NTS + 31) / 32 * 32) + 255) / 256 * 256;
 constexpr long PF_BYTES = PF_PART + 4L * pf::MAX_PSLOTS * NKV * pf::PART_FLOATS;
 static_assert(PF_BAR_BYTES % 4 == 0 && PF_PART % 256 == 0, "prefill workspace alignment");
-static_assert(4L * (64 + 1) * NXCD <= PF_BAR_LINES, "the barrier words fit their lines");
+static_assert(4L * (64 + 32) * NXCD <= PF_BAR_LINES, "the barrier words fit their lines");
 
 // The attention work of a prefill of n positions from position start: query block b (positions
 // start + 32 b ..) reads key blocks 0 .. nkb(b) - 1 (64 keys each, causal), in chunks of
@@ -460,6 +460,29 @@ static int prefill_units(int n, int start, pf::PParams& P) {
   for (int i = 0; i < nu; ++i) P.unit[i] = (unsigned short)(u[i].b | u[i].c << 6 | (u[i].s - 1) << 8);
   P.nunits = nu;
   return QWEN_OK;
+}
+
+// The prefill builds: one-workgroup-per-CU kernels with tiles for at most 16, 64, .. 1024 positions,
+// then the two-workgroups-per-CU kernel for longer prompts
+constexpr int PF_CLASS_MAX[] = {16, 64, 128, 256, 512, 1024};
+constexpr int PF_CLASSES = sizeof(PF_CLASS_MAX) / sizeof(int);
+static_assert(PF_CLASS_MAX[PF_CLASSES - 1] == pf::MID_MAX, "class limits");
+struct PrefillBuild {
+  const void* kernel;
+  int grid, threads;
+};
+PrefillBuild prefill_build(int cls) {
+  static const void* const mid[PF_CLASSES] = {
+      (const void*)pf::qwen_prefill_mid_kernel<16>,  (const void*)pf::qwen_prefill_mid_kernel<64>,
+      (const void*)pf::qwen_prefill_mid_kernel<128>, (const void*)pf::qwen_prefill_mid_kernel<256>,
+      (const void*)pf::qwen_prefill_mid_kernel<512>, (const void*)pf::qwen_prefill_mid_kernel<1024>};
+  if (cls < PF_CLASSES) return {mid[cls], NWG, pf::MNT};
+  return {(const void*)pf::qwen_prefill_kernel, pf::NWG_PF, pf::NT};
+}
+int prefill_class(int n) {
+  int k = 0;
+  while (k < PF_CLASSES && n > PF_CLASS_MAX[k]) ++k;
+  return k;
 }
 
 // sampler buffer: the sampler's work area (two copies, chosen by launch parity)
@@ -675,10 +698,13 @@ extern "C" int qwen_prefill(const int* ids, int n, const void* embed_weight, con
   if (rc != QWEN_OK) return rc;
   if ((rc = heap_workspace(st)) != QWEN_OK) return rc;
   if (!st->pf) {
-    int occ = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, (const void*)pf::qwen_prefill_kernel, pf::NT, 0) !=
-            hipSuccess || occ < pf::WG_PER_CU)
-      return QWEN_ERR_DEVICE;
+    // every build must fit its workgroups per CU (the grids are one round of resident workgroups)
+    for (int k = 0; k <= PF_CLASSES; ++k) {
+      const PrefillBuild b = prefill_build(k);
+      int occ = 0;
+      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, b.kernel, b.threads, 0) != hipSuccess || occ * NWG < b.grid)
+        return QWEN_ERR_DEVICE;
+    }
     void* p = nullptr;
     if (hipMalloc(&p, PF_BYTES) != hipSuccess) return QWEN_ERR_LAUNCH;
     if ((rc = check_placement((const void*)qwen_placement_probe_pf, pf::NWG_PF, pf::NT, (u32*)p, stream)) != QWEN_OK) {
@@ -717,8 +743,8 @@ extern "C" int qwen_prefill(const int* ids, int n, const void* embed_weight, con
   if ((rc = prefill_units(n, start_position, P)) != QWEN_OK) return rc;
   if (zero_words(P.bar, PF_BAR_BYTES, stream) != QWEN_OK) return QWEN_ERR_LAUNCH;
   void* args[] = {&P};
-  if (hipLaunchCooperativeKernel((const void*)pf::qwen_prefill_kernel, dim3(pf::NWG_PF), dim3(pf::NT), args, 0, stream) !=
-      hipSuccess)
+  const PrefillBuild b = prefill_build(prefill_class(n));
+  if (hipLaunchCooperativeKernel(b.kernel, dim3(b.grid), dim3(b.threads), args, 0, stream) != hipSuccess)
     return QWEN_ERR_LAUNCH;
   return QWEN_OK;
 }

@@ -304,6 +304,29 @@ def test_batched_prefill_chunked_equals_whole(ext, full, n, cuts):
     assert torch.equal(a.hidden, b.hidden)
 
 
+@pytest.mark.parametrize("sizes", [(1, 15, 16, 17, 63, 64, 65, 127, 128, 129, 255, 256, 257), (512, 511, 1024), (513, 1023, 511)])
+def test_batched_prefill_builds_agree(ext, full, sizes):
+    """Every prefill build (chosen by a call's length: at most 16, 64, 128, 256, 512, 1024 positions,
+    and longer) at the edges of its range, against the longest prompts' build, which the oracle
+    checks: a prompt prefilled in pieces of these sizes leaves the K/V cache and the hidden state of
+    one prefill of all of it, bit for bit. Run twice: the second pass finds the buffers of the first."""
+    hw, w, packed = full
+    n = sum(sizes)
+    assert n > 1024
+    ids = qw.synthetic_prompt(n, seed=62)
+    a, b = Run(w, packed, 4), Run(w, packed, 4)
+    _prefill(ext, a, ids, 0)
+    for _ in range(2):
+        b.kc.zero_()
+        b.vc.zero_()
+        lo = 0
+        for k in sizes:
+            _prefill(ext, b, ids[lo:lo + k], lo)
+            lo += k
+        assert torch.equal(a.kc, b.kc) and torch.equal(a.vc, b.vc)
+        assert torch.equal(a.hidden, b.hidden)
+
+
 def test_batched_prefill_bad_id_reported(ext, full):
     """An id outside the vocabulary inside a device id tensor is reported by last_error()
     as QWEN_ERR_BAD_TOKEN (5), and the next prefill works."""
