@@ -428,13 +428,13 @@ static_assert(PF_BAR_BYTES % 4 == 0 && PF_PART % 256 == 0, "prefill workspace al
 static_assert(4L * (64 + 32) * NXCD <= PF_BAR_LINES, "the barrier words fit their lines");
 
 // The attention work of a prefill of n positions from position start: query block b (positions
-// start + 32 b ..) reads key blocks 0 .. nkb(b) - 1 (64 keys each, causal), in chunks of
-// pf::KCHUNK key blocks; a block with more than one chunk is split into units (the kernel merges their partial
-// results). Units are sorted longest first (ties: later query block first, then chunk order),
-// the order in which the kernel deals them out.
-static int prefill_units(int n, int start, pf::PParams& P) {
+// start + 32 b ..) reads key blocks 0 .. nkb(b) - 1 (64 keys each, causal), in units of `blocks` key
+// blocks: chunks (pf::KCHUNK) or groups (pf::KSUB), whose results the kernel merges where a query
+// block has several. Units are sorted longest first (ties: later query block first, then key order),
+// the order in which the kernel deals them out. False if they do not fit the tables.
+static bool prefill_units(int n, int start, int blocks, pf::PParams& P) {
   const int nqb = (n + pf::QR - 1) / pf::QR;
-  if (nqb > pf::MAX_QB) return QWEN_ERR_ARG;
+  if (nqb > pf::MAX_QB) return false;
   struct U {
     int cost, b, c, s;
   } u[pf::MAX_UNITS];
@@ -442,24 +442,21 @@ static int prefill_units(int n, int start, pf::PParams& P) {
   for (int b = 0; b < nqb; ++b) {
     const int qmax = (pf::QR * b + pf::QR < n ? pf::QR * b + pf::QR : n) - 1 + start;
     const int nkb = qmax / pf::QB + 1;
-    const int sb = (nkb + pf::KCHUNK - 1) / pf::KCHUNK;
-    if (sb > pf::MAX_CHUNKS || nu + sb > pf::MAX_UNITS) return QWEN_ERR_ARG;
+    const int sb = (nkb + blocks - 1) / blocks;
+    if (sb > pf::MAX_PARTS || nu + sb > pf::MAX_UNITS || (sb > 1 && slot + sb > pf::MAX_PSLOTS)) return false;
     P.pslot[b] = (unsigned char)(sb > 1 ? slot : 0);
     if (sb > 1) slot += sb;
-    for (int c = 0; c < sb; ++c) {
-      const int left = nkb - pf::KCHUNK * c;
-      u[nu++] = {left < pf::KCHUNK ? left : pf::KCHUNK, b, c, sb};
-    }
+    for (int c = 0; c < sb; ++c) u[nu++] = {std::min(blocks, nkb - blocks * c), b, c, sb};
   }
-  if (slot > pf::MAX_PSLOTS) return QWEN_ERR_ARG;
   std::sort(u, u + nu, [](const U& x, const U& y) {
     if (x.cost != y.cost) return x.cost > y.cost;
     if (x.b != y.b) return x.b > y.b;
     return x.c < y.c;
   });
-  for (int i = 0; i < nu; ++i) P.unit[i] = (unsigned short)(u[i].b | u[i].c << 6 | (u[i].s - 1) << 8);
+  for (int i = 0; i < nu; ++i) P.unit[i] = (unsigned short)(u[i].b | u[i].c << 6 | (u[i].s - 1) << 9);
   P.nunits = nu;
-  return QWEN_OK;
+  P.unit_blocks = blocks;
+  return true;
 }
 
 // The prefill builds: one-workgroup-per-CU kernels with tiles for at most 16, 64, .. 1024 positions,
@@ -467,6 +464,7 @@ static int prefill_units(int n, int start, pf::PParams& P) {
 constexpr int PF_CLASS_MAX[] = {16, 64, 128, 256, 512, 1024};
 constexpr int PF_CLASSES = sizeof(PF_CLASS_MAX) / sizeof(int);
 static_assert(PF_CLASS_MAX[PF_CLASSES - 1] == pf::MID_MAX, "class limits");
+constexpr int PF_GROUP_ROUNDS = 1;
 struct PrefillBuild {
   const void* kernel;
   int grid, threads;
@@ -740,10 +738,17 @@ extern "C" int qwen_prefill(const int* ids, int n, const void* embed_weight, con
   P.num_layers = num_layers;
   P.max_seq = max_seq_len;
   P.attn_scale = attn_scale;
-  if ((rc = prefill_units(n, start_position, P)) != QWEN_OK) return rc;
+  const PrefillBuild b = prefill_build(prefill_class(n));
+  if (!prefill_units(n, start_position, pf::KCHUNK, P)) return QWEN_ERR_ARG;
+  if (b.grid == NWG) {
+    pf::PParams S = P;
+    const int nkb = (start_position + n - 1) / pf::QB + 1;  // of the longest key range
+    if ((nkb <= pf::KSUB || nkb > 2 * pf::KSUB) && prefill_units(n, start_position, pf::KSUB, S) &&
+        S.nunits * NKV <= PF_GROUP_ROUNDS * NWG)
+      P = S;
+  }
   if (zero_words(P.bar, PF_BAR_BYTES, stream) != QWEN_OK) return QWEN_ERR_LAUNCH;
   void* args[] = {&P};
-  const PrefillBuild b = prefill_build(prefill_class(n));
   if (hipLaunchCooperativeKernel(b.kernel, dim3(b.grid), dim3(b.threads), args, 0, stream) != hipSuccess)
     return QWEN_ERR_LAUNCH;
   return QWEN_OK;
