@@ -36,6 +36,7 @@
 // 1001-1144 (lm_head + argmax), 1150-1314 (launchers).
 #include <hip/hip_runtime.h>
 #include <hip/hip_fp16.h>
+#include <hip/hip_ext.h>
 
 #include <cstdint>
 #include <cstdio>
@@ -235,6 +236,10 @@ __global__ void qwen_zero_words(u64* p, long n) {
   for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) p[i] = 0;
 }
 
+// the MLP block's one-layer pointer table, from the kernel's arguments: in stream order, where a copy
+// from the host's stack needs the host to wait for it (32 -> 20 us per call)
+__global__ void qwen_write_layer(LDGLayerWeight* tab, LDGLayerWeight layer) { *tab = layer; }
+
 // Exchange workspace of qwen_generate_nosync_noalloc: the same layout as the workspace the
 // other entry points allocate (slots, status line, lm_head pool counters), as module memory,
 // one copy per device. Host code never uses this name as an address: it uses the pointer
@@ -266,6 +271,7 @@ struct DeviceState {
   char* pf = nullptr;             // prefill activations (PF_BYTES), on first use
   char* smp = nullptr;            // the sampler's work area (SMP_BYTES), allocated on first use
   u32 smp_parity = 0;             // sampler launches so far (selects the work area copy)
+  hipEvent_t order = nullptr;     // end of the last launch (see launch_resident)
   u64 clk_khz = 100000;
   u64 deadline = 0;
   u64* trace = nullptr;
@@ -284,10 +290,46 @@ int zero_words(void* p, long bytes, hipStream_t s) {
   return hipGetLastError() == hipSuccess ? QWEN_OK : QWEN_ERR_LAUNCH;
 }
 
-// Every workgroup w of the decode launch (256 x 512) and of the prefill launch (512 x 256) must
-// run on XCD w % 8: the decode's work partition and XCD-local exchange stores, and the prefill's
-// per-XCD barrier (one L2 write-back and invalidate per XCD) rely on it. Checked once per device
-// and geometry with a probe launch that writes into `buf` (n words).
+// The engine's kernels wait for their own workgroups, so all of a launch's must be resident at once:
+// its grid is one round of the chip (one or two workgroups per CU, checked against the occupancy), and
+// no two of these launches may share the chip, nor the device's workspaces. Each launch therefore
+// follows the one before it, on whatever stream: `order` is the event of the last one's end, set by
+// the launch itself (hipExtLaunchKernel), and every call's stream waits for it before its first
+// operation. The runtime's cooperative launch gives the same guarantee by passing through a queue of
+// its own, 18-20 us per call (a sampler launch with nothing to select 27 -> 7 us, the lm_head 78 ->
+// 63); an event recorded after a plain launch costs 3 us more than one that belongs to it. Under
+// stream capture, where an event of outside cannot be waited for, the launch stays a cooperative one.
+bool capturing(hipStream_t stream) {
+  hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(stream, &c) != hipSuccess || c != hipStreamCaptureStatusNone;
+}
+// makes the stream wait for the device's last launch; caller holds g_mu
+int order_after(DeviceState* st, hipStream_t stream) {
+  if (!st->order || capturing(stream)) return QWEN_OK;
+  return hipStreamWaitEvent(stream, st->order, 0) == hipSuccess ? QWEN_OK : QWEN_ERR_LAUNCH;
+}
+// launches a kernel of `grid` workgroups that wait for each other; caller holds g_mu, and the stream
+// has waited for the last launch (order_after)
+int launch_resident(DeviceState* st, const void* kernel, int grid, int threads, void** args, hipStream_t stream) {
+  if (capturing(stream))
+    return hipLaunchCooperativeKernel(kernel, dim3(grid), dim3(threads), args, 0, stream) == hipSuccess ? QWEN_OK
+                                                                                                    : QWEN_ERR_LAUNCH;
+  if (!st->order && hipEventCreateWithFlags(&st->order, hipEventDisableTiming) != hipSuccess) {
+    st->order = nullptr;
+    return QWEN_ERR_LAUNCH;
+  }
+  return hipExtLaunchKernel(kernel, dim3(grid), dim3(threads), args, 0, stream, nullptr, st->order, 0) == hipSuccess
+             ? QWEN_OK
+             : QWEN_ERR_LAUNCH;
+}
+
+// The workgroups w of the decode launch (256 x 512) and of the prefill launches with equal w % 8 must
+// run on one XCD: the decode's work partition and XCD-local exchange stores, and the prefill's per-XCD
+// barrier (one L2 write-back and invalidate per XCD) rely on it ("XCD w % 8" in their comments: which
+// of the chip's XCDs that is does not matter). The dispatcher deals workgroups out in turn, from an XCD
+// that differs from queue to queue and changes when a queue is mapped anew (2400 launches of both
+// geometries, cooperative and plain, between other kernels: always w -> (w + r) % 8, r = 0, 6 or 7).
+// Checked once per device and geometry with a probe launch that writes into `buf` (n words).
 int check_placement(const void* probe, int n, int threads, u32* buf, hipStream_t s) {
   void* args[] = {&buf};
   if (hipLaunchCooperativeKernel(probe, dim3(n), dim3(threads), args, 0, s) != hipSuccess ||
@@ -297,9 +339,9 @@ int check_placement(const void* probe, int n, int threads, u32* buf, hipStream_t
   if (n > 2 * NWG || hipMemcpy(xcc, buf, sizeof(u32) * n, hipMemcpyDeviceToHost) != hipSuccess)
     return QWEN_ERR_LAUNCH;
   for (int w = 0; w < n; ++w)
-    if ((int)(xcc[w] & 15) != xcd_of(w)) {
-      fprintf(stderr, "qwen_megakernel: workgroup %d of %d runs on XCC %u, the kernel needs XCC %d\n", w, n,
-              xcc[w] & 15, xcd_of(w));
+    if ((xcc[w] & 15) != ((xcc[0] & 15) + xcd_of(w)) % NXCD) {
+      fprintf(stderr, "qwen_megakernel: workgroup %d of %d runs on XCC %u, workgroup 0 on %u: not one XCD per w %% 8\n", w, n,
+              xcc[w] & 15, xcc[0] & 15);
       return QWEN_ERR_DEVICE;
     }
   return QWEN_OK;
@@ -368,8 +410,9 @@ int heap_workspace(DeviceState* st) {
 }
 
 // launches the decode kernel on the heap workspace, or (fixed = true) on the device's
-// `scratch` array, in which case nothing is allocated
-int launch(KParams& P, hipStream_t stream, bool fixed = false) {
+// `scratch` array, in which case nothing is allocated. `layer` (the MLP block's): the one-layer pointer
+// table, which the kernel reads from device memory
+int launch(KParams& P, hipStream_t stream, bool fixed = false, const LDGLayerWeight* layer = nullptr) {
   std::lock_guard<std::mutex> lock(g_mu);
   DeviceState* st = nullptr;
   int rc = device_state(&st);
@@ -380,6 +423,13 @@ int launch(KParams& P, hipStream_t stream, bool fixed = false) {
   if (st->trace && (long long)NWG * trace_stages(P.num_layers) * TRACE_EVENTS > st->trace_elems) return QWEN_ERR_ARG;
   // the traced build is the greedy kernel: a sampled launch while tracing would return argmax ids
   if (st->trace && P.sample) return QWEN_ERR_ARG;
+  if ((rc = order_after(st, stream)) != QWEN_OK) return rc;
+  if (layer) {
+    if (!st->tab && hipMalloc(&st->tab, sizeof(LDGLayerWeight)) != hipSuccess) return QWEN_ERR_LAUNCH;
+    hipLaunchKernelGGL(qwen_write_layer, dim3(1), dim3(1), 0, stream, st->tab, *layer);
+    if (hipGetLastError() != hipSuccess) return QWEN_ERR_LAUNCH;
+    P.layers = st->tab;
+  }
   P.ws = w.ws;
   P.status = w.status;
   P.deadline = st->deadline;
@@ -400,9 +450,7 @@ int launch(KParams& P, hipStream_t stream, bool fixed = false) {
                                     : P.top_k > 0      ? (const void*)sampled::qwen_decode_kernel
                                                        : (const void*)tsampled::qwen_decode_kernel)
                                   : (const void*)fast::qwen_decode_kernel;
-  if (hipLaunchCooperativeKernel(kernel, dim3(NWG), dim3(BLOCK), args, 0, stream) != hipSuccess)
-    return QWEN_ERR_LAUNCH;
-  return QWEN_OK;
+  return launch_resident(st, kernel, NWG, BLOCK, args, stream);
 }
 
 // prefill activations for up to MAX_SEQ_LIMIT positions: residual X fp32 [n, 1024], q and the
@@ -520,15 +568,14 @@ int sampler_buffer(DeviceState* st, hipStream_t stream) {
 
 // one sampler launch on the device's work area; caller holds g_mu
 int launch_sampler(DeviceState* st, smp::SParams& S, hipStream_t stream) {
+  int rc = order_after(st, stream);
+  if (rc != QWEN_OK) return rc;
   S.work = (u64*)(st->smp + SMP_WORK);
   S.parity = st->smp_parity++;
   S.status = st->heap.status;
   S.deadline = st->deadline;
   void* args[] = {&S};
-  if (hipLaunchCooperativeKernel((const void*)smp::qwen_sample_kernel, dim3(smp::NB), dim3(smp::NT), args, 0,
-                                 stream) != hipSuccess)
-    return QWEN_ERR_LAUNCH;
-  return QWEN_OK;
+  return launch_resident(st, (const void*)smp::qwen_sample_kernel, smp::NB, smp::NT, args, stream);
 }
 
 int fill_decode(KParams& P, const void* embed, const LDGLayerWeight* lw, const void* fnorm, const void* lm_head,
@@ -747,11 +794,10 @@ extern "C" int qwen_prefill(const int* ids, int n, const void* embed_weight, con
         S.nunits * NKV <= PF_GROUP_ROUNDS * NWG)
       P = S;
   }
+  if ((rc = order_after(st, stream)) != QWEN_OK) return rc;
   if (zero_words(P.bar, PF_BAR_BYTES, stream) != QWEN_OK) return QWEN_ERR_LAUNCH;
   void* args[] = {&P};
-  if (hipLaunchCooperativeKernel(b.kernel, dim3(b.grid), dim3(b.threads), args, 0, stream) != hipSuccess)
-    return QWEN_ERR_LAUNCH;
-  return QWEN_OK;
+  return launch_resident(st, b.kernel, b.grid, b.threads, args, stream);
 }
 
 extern "C" int qwen_prefill_timestamps(unsigned long long* out, int max_entries) {
@@ -874,35 +920,23 @@ extern "C" int qwen_mlp_block(const void* x_f16, const void* post_norm_weight, c
   if (!aligned16(x_f16) || !aligned16(post_norm_weight) || !aligned16(gate_weight) || !aligned16(up_weight) ||
       !aligned16(down_weight) || !aligned16(y_out))
     return QWEN_ERR_ARG;
-  // the kernel reads the layer pointer table from device memory
+  if (capturing(stream)) return QWEN_ERR_LAUNCH;  // (not for stream capture: the table outlives no replay)
   LDGLayerWeight h;
   memset(&h, 0, sizeof(h));
   h.post_attn_layernorm_weight = post_norm_weight;
   h.gate_proj_weight = gate_weight;
   h.up_proj_weight = up_weight;
   h.down_proj_weight = down_weight;
-  LDGLayerWeight* tab = nullptr;
-  {
-    std::lock_guard<std::mutex> lock(g_mu);
-    DeviceState* st = nullptr;
-    int rc = device_state(&st);
-    if (rc != QWEN_OK) return rc;
-    if (!st->tab && hipMalloc(&st->tab, sizeof(LDGLayerWeight)) != hipSuccess) return QWEN_ERR_LAUNCH;
-    tab = st->tab;
-  }
-  if (hipMemcpyAsync(tab, &h, sizeof(h), hipMemcpyHostToDevice, stream) != hipSuccess) return QWEN_ERR_LAUNCH;
-  if (hipStreamSynchronize(stream) != hipSuccess) return QWEN_ERR_LAUNCH;
   KParams P;
   memset(&P, 0, sizeof(P));
   P.eos = -1;
-  P.layers = tab;
   P.in_vec = (const _Float16*)x_f16;
   P.out_vec = y_out;
   P.mode = MODE_MLP;
   P.num_layers = 1;
   P.num_steps = 1;
   P.max_seq = MAX_SEQ_LIMIT;
-  return launch(P, stream);
+  return launch(P, stream, false, &h);
 }
 
 namespace {

@@ -327,6 +327,42 @@ def test_batched_prefill_builds_agree(ext, full, sizes):
         assert torch.equal(a.hidden, b.hidden)
 
 
+def test_calls_on_two_streams_in_turn(ext, full):
+    """The engine's launches share the device's workspaces, and their workgroups wait for each other:
+    each launch follows the one before it on whatever stream. Decode, prefill, sampling and the
+    isolated blocks issued on two streams in turn, with no host synchronisation between them, give
+    what they give alone."""
+    hw, w, packed = full
+    ids = qw.synthetic_prompt(70, seed=63)
+    f = torch.tensor(ids, dtype=torch.int32, device="cuda")
+    x = torch.randn(1024, device="cuda", generator=torch.Generator(device="cuda").manual_seed(5)).half()
+    layer = w["layer_weights"]
+
+    def call(run, lo):
+        ext.prefill(f, w["embed_weight"], packed, w["cos_table"], w["sin_table"], run.kc, run.vc, run.hidden, 2, 0,
+                    MAX_SEQ, SCALE)
+        toks = ext.generate_ex(ids[-1], 4, None, w["embed_weight"], packed, w["final_norm_weight"], w["lm_head_weight"],
+                               w["cos_table"], w["sin_table"], run.kc, run.vc, run.hidden, run.norm_out, lo, None, 2,
+                               70, MAX_SEQ, SCALE)
+        return [run.kc, run.vc, lo, toks, ext.sample(lo[0], 0.8, 0, 0.9, 3, 7), ext.lm_head_argmax(run.hidden, w["lm_head_weight"]),
+                ext.mlp_block(x, layer[7], layer[8], layer[9], layer[10])]
+
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    runs = [Run(w, packed, 2) for _ in range(3)]
+    los = [torch.empty(4, V, dtype=torch.float32, device="cuda") for _ in range(3)]
+    want = call(runs[2], los[2])
+    torch.cuda.synchronize()
+    for _ in range(10):
+        got = []
+        for k in (0, 1):
+            with torch.cuda.stream(streams[k]):
+                got.append(call(runs[k], los[k]))
+        torch.cuda.synchronize()
+        assert ext.last_error() == 0
+        for g in got:
+            assert all(torch.equal(p, q) for p, q in zip(g, want))
+
+
 def test_batched_prefill_bad_id_reported(ext, full):
     """An id outside the vocabulary inside a device id tensor is reported by last_error()
     as QWEN_ERR_BAD_TOKEN (5), and the next prefill works."""
