@@ -244,7 +244,7 @@ int qwen_mlp_block(const void* x_f16, const void* post_norm_weight, const void* 
 /* Synchronizes the current device and returns the device-side error state of
  * the last launches: QWEN_OK, QWEN_ERR_TIMEOUT (a wait exceeded its deadline)
  * or QWEN_ERR_BAD_TOKEN (a forced id out of range); clears it and resets the
- * workspace when set. (Workgroup placement, workgroup w on XCD w % 8, is checked
+ * workspace when set. (Workgroup placement, one XCD per w % 8, is checked
  * once per device when the library first uses it: QWEN_ERR_DEVICE from every
  * entry point if it does not hold.) */
 int qwen_last_error(void);

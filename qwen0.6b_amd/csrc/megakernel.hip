@@ -237,7 +237,7 @@ __global__ void qwen_zero_words(u64* p, long n) {
 }
 
 // the MLP block's one-layer pointer table, from the kernel's arguments: in stream order, where a copy
-// from the host's stack needs the host to wait for it (32 -> 20 us per call)
+// from the host's stack needs the host to wait for it (with the launch order below: 32 -> 16 us per call)
 __global__ void qwen_write_layer(LDGLayerWeight* tab, LDGLayerWeight layer) { *tab = layer; }
 
 // Exchange workspace of qwen_generate_nosync_noalloc: the same layout as the workspace the
@@ -507,11 +507,19 @@ static bool prefill_units(int n, int start, int blocks, pf::PParams& P) {
   return true;
 }
 
-// The prefill builds: one-workgroup-per-CU kernels with tiles for at most 16, 64, .. 1024 positions,
-// then the two-workgroups-per-CU kernel for longer prompts
+// The prefill builds: one-workgroup-per-CU kernels with tiles for at most 16, 64, .. 1024 positions, then
+// the two-workgroups-per-CU kernel for longer prompts. The last line lies where 128-position tiles stop
+// giving one tile per CU (1025 positions are 288 QKV tiles for 256 workgroups): at 999 positions the
+// short build takes 2.35 ms against 2.85, at 1919 a one-workgroup-per-CU build 3.83 against 3.72.
 constexpr int PF_CLASS_MAX[] = {16, 64, 128, 256, 512, 1024};
 constexpr int PF_CLASSES = sizeof(PF_CLASS_MAX) / sizeof(int);
 static_assert(PF_CLASS_MAX[PF_CLASSES - 1] == pf::MID_MAX, "class limits");
+// Attention units are groups rather than chunks where the longest key range is a single group (nothing to
+// merge; 15 positions: 5.4 against 6.4 us per layer) or more than two, and all groups fit one per
+// workgroup: 61 positions after 1400, 11.5 us per layer against 20.8 with chunks; 256 after 500, 10.8
+// against 15.4. With two rounds of groups the merges cost more than the split gains (256 after 1000:
+// 24.5 against 20.9), and ranges of two groups are as fast as chunks shared by the halves of a
+// workgroup, with nothing to publish (500 positions: 11.6 against 11.4; 400: 11.2 against 10.4).
 constexpr int PF_GROUP_ROUNDS = 1;
 struct PrefillBuild {
   const void* kernel;
