@@ -117,6 +117,7 @@ struct KParams {
   // (draw_dist); top_k = 0: `tsampled` (temperature alone)
   int top_k;
   float top_p;
+  LDGLayerWeight own_layer;  // MODE_MLP: the block's weights
 };
 constexpr int TOPK_MAX = 128;  // largest top_k of the `sampled` build
 
@@ -176,6 +177,7 @@ constexpr bool kTrace = false;
 constexpr bool kSample = false;
 constexpr bool kTopK = false;
 constexpr bool kDist = false;
+constexpr bool kOwnLayer = false;
 #include "decode_body.inc"
 }  // namespace fast
 
@@ -184,6 +186,7 @@ constexpr bool kTrace = true;
 constexpr bool kSample = false;
 constexpr bool kTopK = false;
 constexpr bool kDist = false;
+constexpr bool kOwnLayer = false;
 #include "decode_body.inc"
 }  // namespace traced
 
@@ -192,6 +195,7 @@ constexpr bool kTrace = false;
 constexpr bool kSample = true;
 constexpr bool kTopK = true;
 constexpr bool kDist = false;
+constexpr bool kOwnLayer = false;
 #include "decode_body.inc"
 }  // namespace sampled
 
@@ -202,6 +206,7 @@ constexpr bool kTrace = false;
 constexpr bool kSample = true;
 constexpr bool kTopK = true;
 constexpr bool kDist = true;
+constexpr bool kOwnLayer = false;
 #include "decode_body.inc"
 }  // namespace dsampled
 
@@ -212,8 +217,21 @@ constexpr bool kTrace = false;
 constexpr bool kSample = true;
 constexpr bool kTopK = false;
 constexpr bool kDist = false;
+constexpr bool kOwnLayer = false;
 #include "decode_body.inc"
 }  // namespace tsampled
+
+// the isolated MLP block: the greedy build with the one layer's pointers in the arguments (a table in
+// memory took a copy that the host waited for, or a kernel of its own: 15.9 -> 11.1 us per call; the
+// same choice at run time in the greedy build made its tokens 1% slower, by its scalar registers)
+namespace isolated {
+constexpr bool kTrace = false;
+constexpr bool kSample = false;
+constexpr bool kTopK = false;
+constexpr bool kDist = false;
+constexpr bool kOwnLayer = true;
+#include "decode_body.inc"
+}  // namespace isolated
 
 // the batched prefill kernel (namespace pf)
 #include "prefill_body.inc"
@@ -235,10 +253,6 @@ __global__ void __launch_bounds__(pf::NT, pf::WG_PER_CU) qwen_placement_probe_pf
 __global__ void qwen_zero_words(u64* p, long n) {
   for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) p[i] = 0;
 }
-
-// the MLP block's one-layer pointer table, from the kernel's arguments: in stream order, where a copy
-// from the host's stack needs the host to wait for it (with the launch order below: 32 -> 16 us per call)
-__global__ void qwen_write_layer(LDGLayerWeight* tab, LDGLayerWeight layer) { *tab = layer; }
 
 // Exchange workspace of qwen_generate_nosync_noalloc: the same layout as the workspace the
 // other entry points allocate (slots, status line, lm_head pool counters), as module memory,
@@ -267,7 +281,6 @@ struct DeviceState {
   int err = QWEN_OK;
   Workspace heap;                 // hipMalloc'd on first use by the allocating entry points
   Workspace fixed;                // the `scratch` array of this device (no allocation)
-  LDGLayerWeight* tab = nullptr;  // the isolated MLP block's one-layer pointer table
   char* pf = nullptr;             // prefill activations (PF_BYTES), on first use
   char* smp = nullptr;            // the sampler's work area (SMP_BYTES), allocated on first use
   u32 smp_parity = 0;             // sampler launches so far (selects the work area copy)
@@ -281,7 +294,7 @@ struct DeviceState {
 
 std::mutex g_mu;
 DeviceState g_dev[MAX_DEVICES];
-// What the library allocates (workspaces, the MLP block's pointer table, the prefill and
+// What the library allocates (workspaces, the prefill and
 // sampler buffers) is held until the process ends and released with it; no exit handler
 // calls into the HIP runtime.
 
@@ -364,7 +377,8 @@ int device_state(DeviceState** out) {
     }
     // every build of the decode kernel must fit one workgroup per CU
     const void* builds[] = {(const void*)fast::qwen_decode_kernel, (const void*)traced::qwen_decode_kernel,
-                            (const void*)sampled::qwen_decode_kernel, (const void*)tsampled::qwen_decode_kernel};
+                            (const void*)sampled::qwen_decode_kernel, (const void*)tsampled::qwen_decode_kernel,
+                            (const void*)isolated::qwen_decode_kernel};
     for (const void* k : builds) {
       int occ = 0;
       if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k, BLOCK, 0) != hipSuccess || occ < 1) return st.err;
@@ -410,9 +424,8 @@ int heap_workspace(DeviceState* st) {
 }
 
 // launches the decode kernel on the heap workspace, or (fixed = true) on the device's
-// `scratch` array, in which case nothing is allocated. `layer` (the MLP block's): the one-layer pointer
-// table, which the kernel reads from device memory
-int launch(KParams& P, hipStream_t stream, bool fixed = false, const LDGLayerWeight* layer = nullptr) {
+// `scratch` array, in which case nothing is allocated
+int launch(KParams& P, hipStream_t stream, bool fixed = false) {
   std::lock_guard<std::mutex> lock(g_mu);
   DeviceState* st = nullptr;
   int rc = device_state(&st);
@@ -423,13 +436,8 @@ int launch(KParams& P, hipStream_t stream, bool fixed = false, const LDGLayerWei
   if (st->trace && (long long)NWG * trace_stages(P.num_layers) * TRACE_EVENTS > st->trace_elems) return QWEN_ERR_ARG;
   // the traced build is the greedy kernel: a sampled launch while tracing would return argmax ids
   if (st->trace && P.sample) return QWEN_ERR_ARG;
+  if (P.mode == MODE_MLP && capturing(stream)) return QWEN_ERR_LAUNCH;  // (the MLP block never was capturable)
   if ((rc = order_after(st, stream)) != QWEN_OK) return rc;
-  if (layer) {
-    if (!st->tab && hipMalloc(&st->tab, sizeof(LDGLayerWeight)) != hipSuccess) return QWEN_ERR_LAUNCH;
-    hipLaunchKernelGGL(qwen_write_layer, dim3(1), dim3(1), 0, stream, st->tab, *layer);
-    if (hipGetLastError() != hipSuccess) return QWEN_ERR_LAUNCH;
-    P.layers = st->tab;
-  }
   P.ws = w.ws;
   P.status = w.status;
   P.deadline = st->deadline;
@@ -446,6 +454,7 @@ int launch(KParams& P, hipStream_t stream, bool fixed = false, const LDGLayerWei
   w.epoch = (u32)next;
   void* args[] = {&P};
   const void* kernel = P.trace    ? (const void*)traced::qwen_decode_kernel
+                       : P.mode == MODE_MLP ? (const void*)isolated::qwen_decode_kernel
                        : P.sample ? (P.top_k > TOPK_MAX ? (const void*)dsampled::qwen_decode_kernel
                                     : P.top_k > 0      ? (const void*)sampled::qwen_decode_kernel
                                                        : (const void*)tsampled::qwen_decode_kernel)
@@ -928,23 +937,20 @@ extern "C" int qwen_mlp_block(const void* x_f16, const void* post_norm_weight, c
   if (!aligned16(x_f16) || !aligned16(post_norm_weight) || !aligned16(gate_weight) || !aligned16(up_weight) ||
       !aligned16(down_weight) || !aligned16(y_out))
     return QWEN_ERR_ARG;
-  if (capturing(stream)) return QWEN_ERR_LAUNCH;  // (not for stream capture: the table outlives no replay)
-  LDGLayerWeight h;
-  memset(&h, 0, sizeof(h));
-  h.post_attn_layernorm_weight = post_norm_weight;
-  h.gate_proj_weight = gate_weight;
-  h.up_proj_weight = up_weight;
-  h.down_proj_weight = down_weight;
   KParams P;
   memset(&P, 0, sizeof(P));
   P.eos = -1;
+  P.own_layer.post_attn_layernorm_weight = post_norm_weight;
+  P.own_layer.gate_proj_weight = gate_weight;
+  P.own_layer.up_proj_weight = up_weight;
+  P.own_layer.down_proj_weight = down_weight;
   P.in_vec = (const _Float16*)x_f16;
   P.out_vec = y_out;
   P.mode = MODE_MLP;
   P.num_layers = 1;
   P.num_steps = 1;
   P.max_seq = MAX_SEQ_LIMIT;
-  return launch(P, stream, false, &h);
+  return launch(P, stream);
 }
 
 namespace {
