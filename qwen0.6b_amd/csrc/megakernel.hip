@@ -1,4 +1,4 @@
-// Qwen3-0.6B batch-1 decode engine for MI355X (gfx950): one cooperative,
+// Qwen3-0.6B batch-1 decode engine for MI355X (gfx950): one
 // persistent kernel runs whole token steps (embedding, 28 layers, final norm,
 // tied lm_head, argmax) and, in generate mode, feeds each argmax back as the
 // next step's input without returning to the host.
