@@ -303,6 +303,45 @@ int zero_words(void* p, long bytes, hipStream_t s) {
   return hipGetLastError() == hipSuccess ? QWEN_OK : QWEN_ERR_LAUNCH;
 }
 
+// The prefill builds: one-workgroup-per-CU kernels with tiles for at most 16, 64, .. 1024 positions, then
+// the two-workgroups-per-CU kernel for longer prompts. The last line lies where 128-position tiles stop
+// giving one tile per CU (1025 positions are 288 QKV tiles for 256 workgroups): at 999 positions the
+// short build takes 2.35 ms against 2.85, at 1919 a one-workgroup-per-CU build 3.83 against 3.72.
+constexpr int PF_CLASS_MAX[] = {16, 64, 128, 256, 512, 1024};
+constexpr int PF_CLASSES = sizeof(PF_CLASS_MAX) / sizeof(int);
+static_assert(PF_CLASS_MAX[PF_CLASSES - 1] == pf::MID_MAX, "class limits");
+int prefill_class(int n) {
+  int k = 0;
+  while (k < PF_CLASSES && n > PF_CLASS_MAX[k]) ++k;
+  return k;
+}
+
+// Every kernel whose workgroups wait for each other, with the grid it is launched with: one round of the
+// chip's CUs, which all of it must fit at once (device_state checks each; nothing else is launched by
+// launch_resident).
+struct Build {
+  const void* kernel;
+  int grid, threads;
+};
+enum BuildId : int { DEC_GREEDY, DEC_TRACED, DEC_TOPK, DEC_DIST, DEC_TEMP, DEC_MLP, SAMPLER, PREFILL };  // + prefill_class
+const Build BUILDS[] = {
+    {(const void*)fast::qwen_decode_kernel, NWG, BLOCK},
+    {(const void*)traced::qwen_decode_kernel, NWG, BLOCK},
+    {(const void*)sampled::qwen_decode_kernel, NWG, BLOCK},
+    {(const void*)dsampled::qwen_decode_kernel, NWG, BLOCK},
+    {(const void*)tsampled::qwen_decode_kernel, NWG, BLOCK},
+    {(const void*)isolated::qwen_decode_kernel, NWG, BLOCK},
+    {(const void*)smp::qwen_sample_kernel, smp::NB, smp::NT},
+    {(const void*)pf::qwen_prefill_mid_kernel<16>, NWG, pf::MNT},
+    {(const void*)pf::qwen_prefill_mid_kernel<64>, NWG, pf::MNT},
+    {(const void*)pf::qwen_prefill_mid_kernel<128>, NWG, pf::MNT},
+    {(const void*)pf::qwen_prefill_mid_kernel<256>, NWG, pf::MNT},
+    {(const void*)pf::qwen_prefill_mid_kernel<512>, NWG, pf::MNT},
+    {(const void*)pf::qwen_prefill_mid_kernel<1024>, NWG, pf::MNT},
+    {(const void*)pf::qwen_prefill_kernel, pf::NWG_PF, pf::NT},
+};
+static_assert(sizeof(BUILDS) / sizeof(Build) == PREFILL + PF_CLASSES + 1, "a build per prefill class, then the long one");
+
 // The engine's kernels wait for their own workgroups, so all of a launch's must be resident at once:
 // its grid is one round of the chip (one or two workgroups per CU, checked against the occupancy), and
 // no two of these launches may share the chip, nor the device's workspaces. Each launch therefore
@@ -321,17 +360,18 @@ int order_after(DeviceState* st, hipStream_t stream) {
   if (!st->order || capturing(stream)) return QWEN_OK;
   return hipStreamWaitEvent(stream, st->order, 0) == hipSuccess ? QWEN_OK : QWEN_ERR_LAUNCH;
 }
-// launches a kernel of `grid` workgroups that wait for each other; caller holds g_mu, and the stream
-// has waited for the last launch (order_after)
-int launch_resident(DeviceState* st, const void* kernel, int grid, int threads, void** args, hipStream_t stream) {
+// launches one of BUILDS; caller holds g_mu, and the stream has waited for the last launch (order_after)
+int launch_resident(DeviceState* st, int build, void** args, hipStream_t stream) {
+  const Build& b = BUILDS[build];
   if (capturing(stream))
-    return hipLaunchCooperativeKernel(kernel, dim3(grid), dim3(threads), args, 0, stream) == hipSuccess ? QWEN_OK
-                                                                                                    : QWEN_ERR_LAUNCH;
+    return hipLaunchCooperativeKernel(b.kernel, dim3(b.grid), dim3(b.threads), args, 0, stream) == hipSuccess
+               ? QWEN_OK
+               : QWEN_ERR_LAUNCH;
   if (!st->order && hipEventCreateWithFlags(&st->order, hipEventDisableTiming) != hipSuccess) {
     st->order = nullptr;
     return QWEN_ERR_LAUNCH;
   }
-  return hipExtLaunchKernel(kernel, dim3(grid), dim3(threads), args, 0, stream, nullptr, st->order, 0) == hipSuccess
+  return hipExtLaunchKernel(b.kernel, dim3(b.grid), dim3(b.threads), args, 0, stream, nullptr, st->order, 0) == hipSuccess
              ? QWEN_OK
              : QWEN_ERR_LAUNCH;
 }
@@ -375,13 +415,10 @@ int device_state(DeviceState** out) {
               prop.gcnArchName, prop.multiProcessorCount);
       return st.err;
     }
-    // every build of the decode kernel must fit one workgroup per CU
-    const void* builds[] = {(const void*)fast::qwen_decode_kernel, (const void*)traced::qwen_decode_kernel,
-                            (const void*)sampled::qwen_decode_kernel, (const void*)tsampled::qwen_decode_kernel,
-                            (const void*)isolated::qwen_decode_kernel};
-    for (const void* k : builds) {
+    for (const Build& b : BUILDS) {
       int occ = 0;
-      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k, BLOCK, 0) != hipSuccess || occ < 1) return st.err;
+      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, b.kernel, b.threads, 0) != hipSuccess || occ * NWG < b.grid)
+        return st.err;
     }
     int clk_khz = 0;
     if (hipDeviceGetAttribute(&clk_khz, hipDeviceAttributeWallClockRate, dev) != hipSuccess || clk_khz <= 0)
@@ -453,13 +490,11 @@ int launch(KParams& P, hipStream_t stream, bool fixed = false) {
   }
   w.epoch = (u32)next;
   void* args[] = {&P};
-  const void* kernel = P.trace    ? (const void*)traced::qwen_decode_kernel
-                       : P.mode == MODE_MLP ? (const void*)isolated::qwen_decode_kernel
-                       : P.sample ? (P.top_k > TOPK_MAX ? (const void*)dsampled::qwen_decode_kernel
-                                    : P.top_k > 0      ? (const void*)sampled::qwen_decode_kernel
-                                                       : (const void*)tsampled::qwen_decode_kernel)
-                                  : (const void*)fast::qwen_decode_kernel;
-  return launch_resident(st, kernel, NWG, BLOCK, args, stream);
+  const int build = P.trace              ? DEC_TRACED
+                    : P.mode == MODE_MLP ? DEC_MLP
+                    : P.sample           ? (P.top_k > TOPK_MAX ? DEC_DIST : P.top_k > 0 ? DEC_TOPK : DEC_TEMP)
+                                         : DEC_GREEDY;
+  return launch_resident(st, build, args, stream);
 }
 
 // prefill activations for up to MAX_SEQ_LIMIT positions: residual X fp32 [n, 1024], q and the
@@ -516,13 +551,6 @@ static bool prefill_units(int n, int start, int blocks, pf::PParams& P) {
   return true;
 }
 
-// The prefill builds: one-workgroup-per-CU kernels with tiles for at most 16, 64, .. 1024 positions, then
-// the two-workgroups-per-CU kernel for longer prompts. The last line lies where 128-position tiles stop
-// giving one tile per CU (1025 positions are 288 QKV tiles for 256 workgroups): at 999 positions the
-// short build takes 2.35 ms against 2.85, at 1919 a one-workgroup-per-CU build 3.83 against 3.72.
-constexpr int PF_CLASS_MAX[] = {16, 64, 128, 256, 512, 1024};
-constexpr int PF_CLASSES = sizeof(PF_CLASS_MAX) / sizeof(int);
-static_assert(PF_CLASS_MAX[PF_CLASSES - 1] == pf::MID_MAX, "class limits");
 // Attention units are groups rather than chunks where the longest key range is a single group (nothing to
 // merge; 15 positions: 5.4 against 6.4 us per layer) or more than two, and all groups fit one per
 // workgroup: 61 positions after 1400, 11.5 us per layer against 20.8 with chunks; 256 after 500, 10.8
@@ -530,23 +558,6 @@ static_assert(PF_CLASS_MAX[PF_CLASSES - 1] == pf::MID_MAX, "class limits");
 // 24.5 against 20.9), and ranges of two groups are as fast as chunks shared by the halves of a
 // workgroup, with nothing to publish (500 positions: 11.6 against 11.4; 400: 11.2 against 10.4).
 constexpr int PF_GROUP_ROUNDS = 1;
-struct PrefillBuild {
-  const void* kernel;
-  int grid, threads;
-};
-PrefillBuild prefill_build(int cls) {
-  static const void* const mid[PF_CLASSES] = {
-      (const void*)pf::qwen_prefill_mid_kernel<16>,  (const void*)pf::qwen_prefill_mid_kernel<64>,
-      (const void*)pf::qwen_prefill_mid_kernel<128>, (const void*)pf::qwen_prefill_mid_kernel<256>,
-      (const void*)pf::qwen_prefill_mid_kernel<512>, (const void*)pf::qwen_prefill_mid_kernel<1024>};
-  if (cls < PF_CLASSES) return {mid[cls], NWG, pf::MNT};
-  return {(const void*)pf::qwen_prefill_kernel, pf::NWG_PF, pf::NT};
-}
-int prefill_class(int n) {
-  int k = 0;
-  while (k < PF_CLASSES && n > PF_CLASS_MAX[k]) ++k;
-  return k;
-}
 
 // sampler buffer: the sampler's work area (two copies, chosen by launch parity)
 constexpr long SMP_WORK = 0;
@@ -592,7 +603,7 @@ int launch_sampler(DeviceState* st, smp::SParams& S, hipStream_t stream) {
   S.status = st->heap.status;
   S.deadline = st->deadline;
   void* args[] = {&S};
-  return launch_resident(st, (const void*)smp::qwen_sample_kernel, smp::NB, smp::NT, args, stream);
+  return launch_resident(st, SAMPLER, args, stream);
 }
 
 int fill_decode(KParams& P, const void* embed, const LDGLayerWeight* lw, const void* fnorm, const void* lm_head,
@@ -760,13 +771,6 @@ extern "C" int qwen_prefill(const int* ids, int n, const void* embed_weight, con
   if (rc != QWEN_OK) return rc;
   if ((rc = heap_workspace(st)) != QWEN_OK) return rc;
   if (!st->pf) {
-    // every build must fit its workgroups per CU (the grids are one round of resident workgroups)
-    for (int k = 0; k <= PF_CLASSES; ++k) {
-      const PrefillBuild b = prefill_build(k);
-      int occ = 0;
-      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, b.kernel, b.threads, 0) != hipSuccess || occ * NWG < b.grid)
-        return QWEN_ERR_DEVICE;
-    }
     void* p = nullptr;
     if (hipMalloc(&p, PF_BYTES) != hipSuccess) return QWEN_ERR_LAUNCH;
     if ((rc = check_placement((const void*)qwen_placement_probe_pf, pf::NWG_PF, pf::NT, (u32*)p, stream)) != QWEN_OK) {
@@ -802,9 +806,9 @@ extern "C" int qwen_prefill(const int* ids, int n, const void* embed_weight, con
   P.num_layers = num_layers;
   P.max_seq = max_seq_len;
   P.attn_scale = attn_scale;
-  const PrefillBuild b = prefill_build(prefill_class(n));
+  const int cls = prefill_class(n);
   if (!prefill_units(n, start_position, pf::KCHUNK, P)) return QWEN_ERR_ARG;
-  if (b.grid == NWG) {
+  if (cls < PF_CLASSES) {
     pf::PParams S = P;
     const int nkb = (start_position + n - 1) / pf::QB + 1;  // of the longest key range
     if ((nkb <= pf::KSUB || nkb > 2 * pf::KSUB) && prefill_units(n, start_position, pf::KSUB, S) &&
@@ -814,7 +818,7 @@ extern "C" int qwen_prefill(const int* ids, int n, const void* embed_weight, con
   if ((rc = order_after(st, stream)) != QWEN_OK) return rc;
   if (zero_words(P.bar, PF_BAR_BYTES, stream) != QWEN_OK) return QWEN_ERR_LAUNCH;
   void* args[] = {&P};
-  return launch_resident(st, b.kernel, b.grid, b.threads, args, stream);
+  return launch_resident(st, PREFILL + cls, args, stream);
 }
 
 extern "C" int qwen_prefill_timestamps(unsigned long long* out, int max_entries) {
