@@ -349,15 +349,35 @@ static_assert(sizeof(BUILDS) / sizeof(Build) == PREFILL + PF_CLASSES + 1, "a bui
 // the launch itself (hipExtLaunchKernel), and every call's stream waits for it before its first
 // operation. The runtime's cooperative launch gives the same guarantee by passing through a queue of
 // its own, 18-20 us per call (a sampler launch with nothing to select 27 -> 7 us, the lm_head 78 ->
-// 63); an event recorded after a plain launch costs 3 us more than one that belongs to it. Under
-// stream capture, where an event of outside cannot be waited for, the launch stays a cooperative one.
+// 63); an event recorded after a plain launch costs 3 us more than one that belongs to it.
+// A captured call puts the same wait and the same record into the graph, as event nodes, so that each
+// replay waits for the launch before it and later ones wait for the replay (the order is that of the
+// host's calls, hipGraphLaunch among them). Its launch is a cooperative one: replays that several
+// threads launch at once are then still taken one after the other.
 bool capturing(hipStream_t stream) {
   hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
   return hipStreamIsCapturing(stream, &c) != hipSuccess || c != hipStreamCaptureStatusNone;
 }
+// adds a node to the stream's capture that waits for the event, or records it, at every replay
+int capture_event(hipStream_t stream, hipEvent_t event, bool record) {
+  hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
+  unsigned long long id = 0;
+  hipGraph_t graph = nullptr;
+  const hipGraphNode_t* last = nullptr;
+  size_t n = 0;
+  if (hipStreamGetCaptureInfo_v2(stream, &c, &id, &graph, &last, &n) != hipSuccess || c != hipStreamCaptureStatusActive)
+    return QWEN_ERR_LAUNCH;
+  hipGraphNode_t node = nullptr;
+  const hipError_t e = record ? hipGraphAddEventRecordNode(&node, graph, last, n, event)
+                              : hipGraphAddEventWaitNode(&node, graph, last, n, event);
+  return e == hipSuccess &&
+                 hipStreamUpdateCaptureDependencies(stream, &node, 1, hipStreamSetCaptureDependencies) == hipSuccess
+             ? QWEN_OK
+             : QWEN_ERR_LAUNCH;
+}
 // makes the stream wait for the device's last launch; caller holds g_mu
 int order_after(DeviceState* st, hipStream_t stream) {
-  if (!st->order || capturing(stream)) return QWEN_OK;
+  if (capturing(stream)) return capture_event(stream, st->order, /*record=*/false);
   return hipStreamWaitEvent(stream, st->order, 0) == hipSuccess ? QWEN_OK : QWEN_ERR_LAUNCH;
 }
 // launches one of BUILDS; caller holds g_mu, and the stream has waited for the last launch (order_after)
@@ -365,12 +385,8 @@ int launch_resident(DeviceState* st, int build, void** args, hipStream_t stream)
   const Build& b = BUILDS[build];
   if (capturing(stream))
     return hipLaunchCooperativeKernel(b.kernel, dim3(b.grid), dim3(b.threads), args, 0, stream) == hipSuccess
-               ? QWEN_OK
+               ? capture_event(stream, st->order, /*record=*/true)
                : QWEN_ERR_LAUNCH;
-  if (!st->order && hipEventCreateWithFlags(&st->order, hipEventDisableTiming) != hipSuccess) {
-    st->order = nullptr;
-    return QWEN_ERR_LAUNCH;
-  }
   return hipExtLaunchKernel(b.kernel, dim3(b.grid), dim3(b.threads), args, 0, stream, nullptr, st->order, 0) == hipSuccess
              ? QWEN_OK
              : QWEN_ERR_LAUNCH;
@@ -433,7 +449,9 @@ int device_state(DeviceState** out) {
     }
     st.err = check_placement((const void*)qwen_placement_probe, NWG, BLOCK, (u32*)fixed, nullptr);
     if (st.err != QWEN_OK) return st.err;
-    if (zero_words(fixed, WORKSPACE_BYTES, nullptr) != QWEN_OK || hipDeviceSynchronize() != hipSuccess) {
+    if (zero_words(fixed, WORKSPACE_BYTES, nullptr) != QWEN_OK ||
+        hipEventCreateWithFlags(&st.order, hipEventDisableTiming) != hipSuccess ||
+        hipEventRecord(st.order, nullptr) != hipSuccess || hipDeviceSynchronize() != hipSuccess) {
       st.err = QWEN_ERR_LAUNCH;
       return st.err;
     }

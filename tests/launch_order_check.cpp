@@ -44,6 +44,7 @@ struct Stream {
   bool capturing = false, capture_unknown = false;
   uint32_t mask = 0xffffffffu;  // every word of its CU mask
   std::vector<Node> graph;
+  Node pending;  // an explicitly added node, until the capture's dependencies are set to it
 };
 std::recursive_mutex mu;
 std::vector<Op> ops;
@@ -173,21 +174,43 @@ hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
   static int used;
   return *e = (hipEvent_t)(pool + used++), hipSuccess;
 }
-hipError_t hipEventRecordWithFlags(hipEvent_t e, hipStream_t s, unsigned flags) {
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
   LOCK;
-  Stream& t = streams[s];
-  if (t.capturing && flags != hipEventRecordExternal) return hipErrorStreamCaptureIsolation;  // (would not order outside)
-  if (t.capturing) t.graph.push_back({Node::RECORD, "record", false, e});
-  else events[e] = add(s, "record", false, false);
+  if (streams[s].capturing) return hipErrorStreamCaptureIsolation;  // (orders nothing outside the graph)
+  events[e] = add(s, "record", false, false);
   return hipSuccess;
 }
-hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) { return hipEventRecordWithFlags(e, s, 0); }
-hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned flags) {
+hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned) {
   LOCK;
-  Stream& t = streams[s];
-  if (t.capturing && flags != hipEventWaitExternal) return hipErrorStreamCaptureIsolation;
-  if (t.capturing) t.graph.push_back({Node::WAIT, "wait", false, e});
-  else add(s, "wait", false, false, events.count(e) ? events[e] : -1);
+  if (streams[s].capturing) return hipErrorStreamCaptureIsolation;
+  add(s, "wait", false, false, events.count(e) ? events[e] : -1);
+  return hipSuccess;
+}
+// (a captured stream stands for its graph; its nodes are one chain)
+hipError_t hipStreamGetCaptureInfo_v2(hipStream_t s, hipStreamCaptureStatus* st, unsigned long long* id, hipGraph_t* g,
+                                      const hipGraphNode_t** deps, size_t* n) {
+  LOCK;
+  *st = streams[s].capturing ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
+  *id = 1, *g = (hipGraph_t)s, *deps = nullptr, *n = streams[s].graph.size();
+  return hipSuccess;
+}
+hipError_t hipGraphAddEventWaitNode(hipGraphNode_t* node, hipGraph_t g, const hipGraphNode_t*, size_t n, hipEvent_t e) {
+  LOCK;
+  if (n != streams[(hipStream_t)g].graph.size()) return hipErrorInvalidValue;
+  if (!events.count(e)) complain("a node waits for an event that was never recorded");
+  streams[(hipStream_t)g].pending = {Node::WAIT, "wait", false, e};
+  return *node = (hipGraphNode_t)g, hipSuccess;
+}
+hipError_t hipGraphAddEventRecordNode(hipGraphNode_t* node, hipGraph_t g, const hipGraphNode_t*, size_t n, hipEvent_t e) {
+  LOCK;
+  if (n != streams[(hipStream_t)g].graph.size()) return hipErrorInvalidValue;
+  streams[(hipStream_t)g].pending = {Node::RECORD, "record", false, e};
+  return *node = (hipGraphNode_t)g, hipSuccess;
+}
+hipError_t hipStreamUpdateCaptureDependencies(hipStream_t s, hipGraphNode_t* node, size_t n, unsigned flags) {
+  LOCK;
+  if (n != 1 || *node != (hipGraphNode_t)s || flags != hipStreamSetCaptureDependencies) return hipErrorInvalidValue;
+  streams[s].graph.push_back(streams[s].pending);
   return hipSuccess;
 }
 hipError_t hipLaunchKernel(const void* k, dim3, dim3, void**, size_t, hipStream_t s) {

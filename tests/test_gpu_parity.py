@@ -363,6 +363,53 @@ def test_calls_on_two_streams_in_turn(ext, full):
             assert all(torch.equal(p, q) for p, q in zip(g, want))
 
 
+def test_replayed_prefill_beside_eager_calls(ext, full):
+    """A captured prefill follows the eager launch before it and later ones follow the replay, on another
+    stream and with no host synchronisation between them: every replay leaves the cache and the hidden
+    state of the same prefill made eagerly, and the eager calls give what they give alone. The replays
+    read other ids each time (the graph holds the id tensor, not its values)."""
+    hw, w, packed = full
+    rounds, ids = 4, torch.tensor(qw.synthetic_prompt(61, seed=64), dtype=torch.int32, device="cuda")
+    prompts = [ids.roll(k).contiguous() for k in range(rounds)]
+    a, b, e = Run(w, packed, 2), Run(w, packed, 2), Run(w, packed, 2)
+
+    def prefill(run, t):
+        ext.prefill(t, w["embed_weight"], packed, w["cos_table"], w["sin_table"], run.kc, run.vc, run.hidden, 2, 0,
+                    MAX_SEQ, SCALE)
+
+    def eager():
+        prefill(e, prompts[0])
+        toks = ext.generate_ex(5, 4, None, w["embed_weight"], packed, w["final_norm_weight"], w["lm_head_weight"],
+                               w["cos_table"], w["sin_table"], e.kc, e.vc, e.hidden, e.norm_out, None, None, 2, 61,
+                               MAX_SEQ, SCALE)
+        return [toks, ext.lm_head_argmax(e.hidden, w["lm_head_weight"])]
+
+    want_eager = eager()
+    want = []
+    for t in prompts:
+        prefill(a, t)
+        want.append([x.clone() for x in (a.kc, a.vc, a.hidden)])
+    torch.cuda.synchronize()
+    side, graph, fed = torch.cuda.Stream(), torch.cuda.CUDAGraph(), ids.clone()
+    with torch.cuda.graph(graph, stream=side):
+        prefill(b, fed)
+    torch.cuda.synchronize()
+    got, got_eager = [], []
+    for t in prompts:
+        got_eager.append(eager())
+        with torch.cuda.stream(side):
+            fed.copy_(t)
+            graph.replay()
+            got.append([x.clone() for x in (b.kc, b.vc, b.hidden)])
+        got_eager.append(eager())
+    torch.cuda.synchronize()
+    assert ext.last_error() == 0
+    for g, x in zip(got, want):
+        assert all(torch.equal(p, q) for p, q in zip(g, x))
+    for g in got_eager:
+        assert all(torch.equal(p, q) for p, q in zip(g, want_eager))
+
+
 def test_batched_prefill_bad_id_reported(ext, full):
     """An id outside the vocabulary inside a device id tensor is reported by last_error()
     as QWEN_ERR_BAD_TOKEN (5), and the next prefill works."""

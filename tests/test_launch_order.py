@@ -35,6 +35,12 @@ def test_calls_follow_each_other(check, scenario):
     check(scenario)
 
 
+def test_captured_calls_are_ordered(check):
+    """A replay of captured calls waits for the eager launch before it and is waited for by the next, on
+    whatever streams, the first time and later."""
+    check("captured")
+
+
 @pytest.mark.parametrize("build", ["4fast", "6traced", "7sampled", "8dsampled", "8tsampled", "8isolated", "qwen_sample_kernel",
                                    "mid_kernelILi16E", "mid_kernelILi64E", "mid_kernelILi128E", "mid_kernelILi256E",
                                    "mid_kernelILi512E", "mid_kernelILi1024E", "19qwen_prefill_kernel"])
