@@ -380,13 +380,26 @@ int order_after(DeviceState* st, hipStream_t stream) {
   if (capturing(stream)) return capture_event(stream, st->order, /*record=*/false);
   return hipStreamWaitEvent(stream, st->order, 0) == hipSuccess ? QWEN_OK : QWEN_ERR_LAUNCH;
 }
+// false for a stream whose queue is restricted to some of the CUs (hipExtStreamCreateWithCUMask): a grid
+// that needs all of them never gets resident there. The cooperative queue, which such a stream's
+// launches then pass through, is not restricted (the question costs 0.2 us per call).
+bool whole_chip(hipStream_t stream) {
+  u32 mask[NWG / 32] = {};
+  if (hipExtStreamGetCUMask(stream, NWG / 32, mask) != hipSuccess) return false;
+  for (u32 m : mask)
+    if (m != 0xffffffffu) return false;
+  return true;
+}
 // launches one of BUILDS; caller holds g_mu, and the stream has waited for the last launch (order_after)
 int launch_resident(DeviceState* st, int build, void** args, hipStream_t stream) {
   const Build& b = BUILDS[build];
-  if (capturing(stream))
-    return hipLaunchCooperativeKernel(b.kernel, dim3(b.grid), dim3(b.threads), args, 0, stream) == hipSuccess
-               ? capture_event(stream, st->order, /*record=*/true)
-               : QWEN_ERR_LAUNCH;
+  const bool captured = capturing(stream);
+  if (captured || !whole_chip(stream)) {
+    if (hipLaunchCooperativeKernel(b.kernel, dim3(b.grid), dim3(b.threads), args, 0, stream) != hipSuccess)
+      return QWEN_ERR_LAUNCH;
+    if (captured) return capture_event(stream, st->order, /*record=*/true);
+    return hipEventRecord(st->order, stream) == hipSuccess ? QWEN_OK : QWEN_ERR_LAUNCH;
+  }
   return hipExtLaunchKernel(b.kernel, dim3(b.grid), dim3(b.threads), args, 0, stream, nullptr, st->order, 0) == hipSuccess
              ? QWEN_OK
              : QWEN_ERR_LAUNCH;

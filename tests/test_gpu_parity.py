@@ -410,6 +410,38 @@ def test_replayed_prefill_beside_eager_calls(ext, full):
         assert all(torch.equal(p, q) for p, q in zip(g, want_eager))
 
 
+def test_stream_with_a_cu_mask(ext, full):
+    """Calls on a stream restricted to a quarter of the CUs: the grids need the whole chip, and the calls
+    give what they give on any stream."""
+    hw, w, packed = full
+    torch.cuda.synchronize()
+    loaded = next(line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line)
+    hip = ctypes.CDLL(loaded)
+    mask, s = (ctypes.c_uint32 * 8)(*[0x000000FF] * 8), ctypes.c_void_p()
+    assert hip.hipExtStreamCreateWithCUMask(ctypes.byref(s), 8, mask) == 0
+    ids = torch.tensor(qw.synthetic_prompt(40, seed=65), dtype=torch.int32, device="cuda")
+
+    def calls(run):
+        ext.prefill(ids, w["embed_weight"], packed, w["cos_table"], w["sin_table"], run.kc, run.vc, run.hidden, 2, 0,
+                    MAX_SEQ, SCALE)
+        lo = torch.empty(2, V, dtype=torch.float32, device="cuda")
+        toks = ext.generate_ex(5, 2, None, w["embed_weight"], packed, w["final_norm_weight"], w["lm_head_weight"],
+                               w["cos_table"], w["sin_table"], run.kc, run.vc, run.hidden, run.norm_out, lo, None, 2, 40,
+                               MAX_SEQ, SCALE)
+        return [run.kc, run.vc, lo, toks, ext.sample(lo[0], 0.8, 0, 0.9, 3, 7)]
+
+    want = calls(Run(w, packed, 2))
+    run = Run(w, packed, 2)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(torch.cuda.ExternalStream(s.value)):
+        got = calls(run)
+    again = calls(Run(w, packed, 2))
+    torch.cuda.synchronize()
+    assert ext.last_error() == 0
+    assert all(torch.equal(p, q) for p, q in zip(got, want))
+    assert all(torch.equal(p, q) for p, q in zip(again, want))
+
+
 def test_batched_prefill_bad_id_reported(ext, full):
     """An id outside the vocabulary inside a device id tensor is reported by last_error()
     as QWEN_ERR_BAD_TOKEN (5), and the next prefill works."""

@@ -41,6 +41,12 @@ def test_captured_calls_are_ordered(check):
     check("captured")
 
 
+def test_streams_with_a_cu_mask(check):
+    """Calls on a stream that is restricted to some CUs: their grids, which need the whole chip, do not go
+    to its queue, and they keep their place in the order."""
+    check("masked")
+
+
 @pytest.mark.parametrize("build", ["4fast", "6traced", "7sampled", "8dsampled", "8tsampled", "8isolated", "qwen_sample_kernel",
                                    "mid_kernelILi16E", "mid_kernelILi64E", "mid_kernelILi128E", "mid_kernelILi256E",
                                    "mid_kernelILi512E", "mid_kernelILi1024E", "19qwen_prefill_kernel"])
