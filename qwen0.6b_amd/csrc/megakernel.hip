@@ -354,9 +354,14 @@ static_assert(sizeof(BUILDS) / sizeof(Build) == PREFILL + PF_CLASSES + 1, "a bui
 // replay waits for the launch before it and later ones wait for the replay (the order is that of the
 // host's calls, hipGraphLaunch among them). Its launch is a cooperative one: replays that several
 // threads launch at once are then still taken one after the other.
-bool capturing(hipStream_t stream) {
+
+// Whether the stream is being captured. Where the runtime cannot say (or the capture has failed) nothing
+// may be sent to the stream: a launch taken for a captured one would be in no order.
+int capture_state(hipStream_t stream, bool* captured) {
   hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
-  return hipStreamIsCapturing(stream, &c) != hipSuccess || c != hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &c) != hipSuccess || c == hipStreamCaptureStatusInvalidated) return QWEN_ERR_LAUNCH;
+  *captured = c == hipStreamCaptureStatusActive;
+  return QWEN_OK;
 }
 // adds a node to the stream's capture that waits for the event, or records it, at every replay
 int capture_event(hipStream_t stream, hipEvent_t event, bool record) {
@@ -376,8 +381,8 @@ int capture_event(hipStream_t stream, hipEvent_t event, bool record) {
              : QWEN_ERR_LAUNCH;
 }
 // makes the stream wait for the device's last launch; caller holds g_mu
-int order_after(DeviceState* st, hipStream_t stream) {
-  if (capturing(stream)) return capture_event(stream, st->order, /*record=*/false);
+int order_after(DeviceState* st, hipStream_t stream, bool captured) {
+  if (captured) return capture_event(stream, st->order, /*record=*/false);
   return hipStreamWaitEvent(stream, st->order, 0) == hipSuccess ? QWEN_OK : QWEN_ERR_LAUNCH;
 }
 // false for a stream whose queue is restricted to some of the CUs (hipExtStreamCreateWithCUMask): a grid
@@ -391,9 +396,8 @@ bool whole_chip(hipStream_t stream) {
   return true;
 }
 // launches one of BUILDS; caller holds g_mu, and the stream has waited for the last launch (order_after)
-int launch_resident(DeviceState* st, int build, void** args, hipStream_t stream) {
+int launch_resident(DeviceState* st, int build, void** args, hipStream_t stream, bool captured) {
   const Build& b = BUILDS[build];
-  const bool captured = capturing(stream);
   if (captured || !whole_chip(stream)) {
     if (hipLaunchCooperativeKernel(b.kernel, dim3(b.grid), dim3(b.threads), args, 0, stream) != hipSuccess)
       return QWEN_ERR_LAUNCH;
@@ -504,8 +508,10 @@ int launch(KParams& P, hipStream_t stream, bool fixed = false) {
   if (st->trace && (long long)NWG * trace_stages(P.num_layers) * TRACE_EVENTS > st->trace_elems) return QWEN_ERR_ARG;
   // the traced build is the greedy kernel: a sampled launch while tracing would return argmax ids
   if (st->trace && P.sample) return QWEN_ERR_ARG;
-  if (P.mode == MODE_MLP && capturing(stream)) return QWEN_ERR_LAUNCH;  // (the MLP block never was capturable)
-  if ((rc = order_after(st, stream)) != QWEN_OK) return rc;
+  bool captured = false;
+  if ((rc = capture_state(stream, &captured)) != QWEN_OK) return rc;
+  if (P.mode == MODE_MLP && captured) return QWEN_ERR_LAUNCH;  // (the MLP block never was capturable)
+  if ((rc = order_after(st, stream, captured)) != QWEN_OK) return rc;
   P.ws = w.ws;
   P.status = w.status;
   P.deadline = st->deadline;
@@ -525,7 +531,7 @@ int launch(KParams& P, hipStream_t stream, bool fixed = false) {
                     : P.mode == MODE_MLP ? DEC_MLP
                     : P.sample           ? (P.top_k > TOPK_MAX ? DEC_DIST : P.top_k > 0 ? DEC_TOPK : DEC_TEMP)
                                          : DEC_GREEDY;
-  return launch_resident(st, build, args, stream);
+  return launch_resident(st, build, args, stream, captured);
 }
 
 // prefill activations for up to MAX_SEQ_LIMIT positions: residual X fp32 [n, 1024], q and the
@@ -627,14 +633,15 @@ int sampler_buffer(DeviceState* st, hipStream_t stream) {
 
 // one sampler launch on the device's work area; caller holds g_mu
 int launch_sampler(DeviceState* st, smp::SParams& S, hipStream_t stream) {
-  int rc = order_after(st, stream);
-  if (rc != QWEN_OK) return rc;
+  bool captured = false;
+  int rc = capture_state(stream, &captured);
+  if (rc != QWEN_OK || (rc = order_after(st, stream, captured)) != QWEN_OK) return rc;
   S.work = (u64*)(st->smp + SMP_WORK);
   S.parity = st->smp_parity++;
   S.status = st->heap.status;
   S.deadline = st->deadline;
   void* args[] = {&S};
-  return launch_resident(st, SAMPLER, args, stream);
+  return launch_resident(st, SAMPLER, args, stream, captured);
 }
 
 int fill_decode(KParams& P, const void* embed, const LDGLayerWeight* lw, const void* fnorm, const void* lm_head,
@@ -846,10 +853,11 @@ extern "C" int qwen_prefill(const int* ids, int n, const void* embed_weight, con
         S.nunits * NKV <= PF_GROUP_ROUNDS * NWG)
       P = S;
   }
-  if ((rc = order_after(st, stream)) != QWEN_OK) return rc;
+  bool captured = false;
+  if ((rc = capture_state(stream, &captured)) != QWEN_OK || (rc = order_after(st, stream, captured)) != QWEN_OK) return rc;
   if (zero_words(P.bar, PF_BAR_BYTES, stream) != QWEN_OK) return QWEN_ERR_LAUNCH;
   void* args[] = {&P};
-  return launch_resident(st, PREFILL + cls, args, stream);
+  return launch_resident(st, PREFILL + cls, args, stream, captured);
 }
 
 extern "C" int qwen_prefill_timestamps(unsigned long long* out, int max_entries) {

@@ -47,6 +47,11 @@ def test_streams_with_a_cu_mask(check):
     check("masked")
 
 
+def test_stream_whose_capture_state_is_unknown(check):
+    """Where the runtime cannot say whether a stream is captured, nothing is sent to it."""
+    check("unknown")
+
+
 @pytest.mark.parametrize("build", ["4fast", "6traced", "7sampled", "8dsampled", "8tsampled", "8isolated", "qwen_sample_kernel",
                                    "mid_kernelILi16E", "mid_kernelILi64E", "mid_kernelILi128E", "mid_kernelILi256E",
                                    "mid_kernelILi512E", "mid_kernelILi1024E", "19qwen_prefill_kernel"])
