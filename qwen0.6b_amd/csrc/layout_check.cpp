@@ -6,6 +6,7 @@
 // covers every context. Exit status 0 = all checks passed.
 #include <cstdio>
 #include <cstdlib>
+#include <cstring>
 #include <vector>
 
 #include "qwen_layout.h"
@@ -27,7 +28,56 @@ static int g_fail = 0;
 
 static bool in_buf(long slot, long off, long n) { return slot >= off && slot < off + n; }
 
-int main() {
+// every key block of every query block is in one unit of the plan, split items have slots of their own,
+// and the units are in the order and the limits that the kernel deals them out by; the part counts it has
+static unsigned check_plan(int n, int start) {
+  PfPlan P;
+  CHECK(pf_plan(n, start, P), "prefill plan of %d at %d refused", n, start);
+  CHECK(P.unit_blocks == PF_KSUB || P.unit_blocks == PF_KCHUNK, "unit size of %d at %d", n, start);
+  const bool groups = P.unit_blocks == PF_KSUB;
+  CHECK(P.nunits > 0 && P.nunits <= PF_MAX_UNITS && (!groups || (n <= PF_MID_MAX && P.nunits * NKV <= NWG)),
+        "%d units for %d at %d", P.nunits, n, start);
+  const int nqb = (n + PF_QR - 1) / PF_QR;
+  std::vector<unsigned> seen(nqb, 0u);  // units of each query block, by number
+  std::vector<int> parts(nqb, 0);
+  std::vector<char> slot(PF_MAX_PSLOTS, 0);
+  unsigned counts = 0;
+  int before = PF_KCHUNK;
+  for (int i = 0; i < P.nunits; ++i) {
+    const PfUnit u = pf_unit(P.unit[i]);
+    CHECK(u.b < nqb, "query block %d of %d at %d", u.b, n, start);
+    if (u.b >= nqb) return counts;
+    const int nkb = pf_key_blocks(n, start, u.b), nb = std::min(P.unit_blocks, nkb - P.unit_blocks * u.c);
+    CHECK(u.s == (nkb + P.unit_blocks - 1) / P.unit_blocks && u.c < u.s && nb > 0 && nb <= before,
+          "unit %d (%d %d %d) of %d at %d", i, u.b, u.c, u.s, n, start);
+    CHECK(!(seen[u.b] >> u.c & 1u), "unit %d of query block %d twice, %d at %d", u.c, u.b, n, start);
+    before = nb;
+    seen[u.b] |= 1u << u.c;
+    parts[u.b] = u.s;
+    counts |= 1u << u.s;
+  }
+  for (int b = 0; b < nqb; ++b) {
+    CHECK(parts[b] > 0 && seen[b] == (1u << parts[b]) - 1u, "query block %d of %d at %d is not covered", b, n, start);
+    for (int c = 0; parts[b] > 1 && c < parts[b]; ++c) {
+      const int k = P.pslot[b] + c;
+      CHECK(k < PF_MAX_PSLOTS && !slot[k < PF_MAX_PSLOTS ? k : 0], "partial slot %d, %d at %d", k, n, start);
+      if (k < PF_MAX_PSLOTS) slot[k] = 1;
+    }
+  }
+  return counts;
+}
+
+int main(int argc, char** argv) {
+  if (argc == 4 && !strcmp(argv[1], "plan")) {  // plan n start: unit size, then the part counts of its items
+    PfPlan P;
+    if (!pf_plan(atoi(argv[2]), atoi(argv[3]), P)) return 1;
+    const unsigned counts = check_plan(atoi(argv[2]), atoi(argv[3]));
+    printf("%d", P.unit_blocks);
+    for (int s = 1; s <= PF_MAX_PARTS; ++s)
+      if (counts >> s & 1u) printf(" %d", s);
+    printf("\n");
+    return g_fail != 0;
+  }
   // ---- exchange layout: buffers contiguous, pair-aligned, inside the workspace ----
   const long offs[] = {B_X, B_QKV, B_PART, B_ATTO, B_OP, B_ACT, B_INT, B_DP, XCD_SLOTS};
   const long sizes[] = {X_SLOTS, QKV_SLOTS, PART_SLOTS, ATTO_SLOTS, OP_SLOTS, ACT_SLOTS, INT_SLOTS, DP_SLOTS};
@@ -492,6 +542,12 @@ int main() {
             CHECK(!distinct(un, 16), "V^T natural order would not conflict (the check would be vacuous)");
           }
   }
+
+  // ---- prefill attention plans: all lengths from some starts, some lengths from all starts ----
+  for (int start : {0, 1, 63, 64, 250, 255, 256, 511, 512, 513, 1000, 1023, 1024, 1400, 1700, 2000, 2046, 2047})
+    for (int n = 1; start + n <= MAX_SEQ_LIMIT; ++n) check_plan(n, start);
+  for (int n : {1, 7, 15, 16, 17, 31, 32, 33, 61, 64, 65, 100, 128, 129, 200, 256, 257, 500, 512, 513, 999, 1024, 1025, 1500})
+    for (int start = 0; start + n <= MAX_SEQ_LIMIT; ++start) check_plan(n, start);
 
   // ---- 64-bit pointers through the 32-bit lane broadcast (readfirstlane: int -> int) ----
   // Device addresses whose low word has bit 31 set are where a signed broadcast result,

@@ -309,7 +309,7 @@ int zero_words(void* p, long bytes, hipStream_t s) {
 // short build takes 2.35 ms against 2.85, at 1919 a one-workgroup-per-CU build 3.83 against 3.72.
 constexpr int PF_CLASS_MAX[] = {16, 64, 128, 256, 512, 1024};
 constexpr int PF_CLASSES = sizeof(PF_CLASS_MAX) / sizeof(int);
-static_assert(PF_CLASS_MAX[PF_CLASSES - 1] == pf::MID_MAX, "class limits");
+static_assert(PF_CLASS_MAX[PF_CLASSES - 1] == PF_MID_MAX, "class limits");
 int prefill_class(int n) {
   int k = 0;
   while (k < PF_CLASSES && n > PF_CLASS_MAX[k]) ++k;
@@ -555,46 +555,6 @@ constexpr long PF_PART = (PF_TS + 8L * ((PF_NTS + 31) / 32 * 32) + 255) / 256 * 
 constexpr long PF_BYTES = PF_PART + 4L * pf::MAX_PSLOTS * NKV * pf::PART_FLOATS;
 static_assert(PF_BAR_BYTES % 4 == 0 && PF_PART % 256 == 0, "prefill workspace alignment");
 static_assert(4L * (64 + 32) * NXCD <= PF_BAR_LINES, "the barrier words fit their lines");
-
-// The attention work of a prefill of n positions from position start: query block b (positions
-// start + 32 b ..) reads key blocks 0 .. nkb(b) - 1 (64 keys each, causal), in units of `blocks` key
-// blocks: chunks (pf::KCHUNK) or groups (pf::KSUB), whose results the kernel merges where a query
-// block has several. Units are sorted longest first (ties: later query block first, then key order),
-// the order in which the kernel deals them out. False if they do not fit the tables.
-static bool prefill_units(int n, int start, int blocks, pf::PParams& P) {
-  const int nqb = (n + pf::QR - 1) / pf::QR;
-  if (nqb > pf::MAX_QB) return false;
-  struct U {
-    int cost, b, c, s;
-  } u[pf::MAX_UNITS];
-  int nu = 0, slot = 0;
-  for (int b = 0; b < nqb; ++b) {
-    const int qmax = (pf::QR * b + pf::QR < n ? pf::QR * b + pf::QR : n) - 1 + start;
-    const int nkb = qmax / pf::QB + 1;
-    const int sb = (nkb + blocks - 1) / blocks;
-    if (sb > pf::MAX_PARTS || nu + sb > pf::MAX_UNITS || (sb > 1 && slot + sb > pf::MAX_PSLOTS)) return false;
-    P.pslot[b] = (unsigned char)(sb > 1 ? slot : 0);
-    if (sb > 1) slot += sb;
-    for (int c = 0; c < sb; ++c) u[nu++] = {std::min(blocks, nkb - blocks * c), b, c, sb};
-  }
-  std::sort(u, u + nu, [](const U& x, const U& y) {
-    if (x.cost != y.cost) return x.cost > y.cost;
-    if (x.b != y.b) return x.b > y.b;
-    return x.c < y.c;
-  });
-  for (int i = 0; i < nu; ++i) P.unit[i] = (unsigned short)(u[i].b | u[i].c << 6 | (u[i].s - 1) << 9);
-  P.nunits = nu;
-  P.unit_blocks = blocks;
-  return true;
-}
-
-// Attention units are groups rather than chunks where the longest key range is a single group (nothing to
-// merge; 15 positions: 5.4 against 6.4 us per layer) or more than two, and all groups fit one per
-// workgroup: 61 positions after 1400, 11.5 us per layer against 20.8 with chunks; 256 after 500, 10.8
-// against 15.4. With two rounds of groups the merges cost more than the split gains (256 after 1000:
-// 24.5 against 20.9), and ranges of two groups are as fast as chunks shared by the halves of a
-// workgroup, with nothing to publish (500 positions: 11.6 against 11.4; 400: 11.2 against 10.4).
-constexpr int PF_GROUP_ROUNDS = 1;
 
 // sampler buffer: the sampler's work area (two copies, chosen by launch parity)
 constexpr long SMP_WORK = 0;
@@ -845,14 +805,7 @@ extern "C" int qwen_prefill(const int* ids, int n, const void* embed_weight, con
   P.max_seq = max_seq_len;
   P.attn_scale = attn_scale;
   const int cls = prefill_class(n);
-  if (!prefill_units(n, start_position, pf::KCHUNK, P)) return QWEN_ERR_ARG;
-  if (cls < PF_CLASSES) {
-    pf::PParams S = P;
-    const int nkb = (start_position + n - 1) / pf::QB + 1;  // of the longest key range
-    if ((nkb <= pf::KSUB || nkb > 2 * pf::KSUB) && prefill_units(n, start_position, pf::KSUB, S) &&
-        S.nunits * NKV <= PF_GROUP_ROUNDS * NWG)
-      P = S;
-  }
+  if (!pf_plan(n, start_position, P.plan)) return QWEN_ERR_ARG;
   bool captured = false;
   if ((rc = capture_state(stream, &captured)) != QWEN_OK || (rc = order_after(st, stream, captured)) != QWEN_OK) return rc;
   if (zero_words(P.bar, PF_BAR_BYTES, stream) != QWEN_OK) return QWEN_ERR_LAUNCH;

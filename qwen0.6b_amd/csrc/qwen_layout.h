@@ -26,6 +26,8 @@
 // stage weights and K/V rows into a ring of 1 KB lines in LDS.
 #pragma once
 
+#include <algorithm>
+
 #ifdef __HIPCC__
 #define QL_HD __host__ __device__ __forceinline__
 #else
@@ -312,6 +314,76 @@ QL_HD int pf_swz8(int r) { return ((r >> 1) & 7) ^ ((r & 1) << 2); }
 // pf_kpos(p, r))
 QL_HD int pf_kpos(int q, int r) { return q ^ (r & 15); }
 QL_HD int pf_vpos(int q, int r) { return q ^ (2 * (r & 7)); }
+
+// ---- prefill attention plan ------------------------------------------------------------
+// Query block b of a call (positions start + 32 b ..) reads key blocks 0 .. nkb(b) - 1 (64 keys each,
+// causal). A query's keys are summed in groups of PF_KSUB blocks (256 keys), the groups' results folded
+// in order into a chunk of PF_KCHUNK blocks (1024 keys), the chunks merged in order: fixed key positions,
+// so the same bits in every launch. A work unit of the kernel is a chunk, or a group where that is faster.
+constexpr int PF_QB = 64;      // keys per block
+constexpr int PF_QR = 32;      // query positions per item
+constexpr int PF_KSUB = 4;     // key blocks per group
+constexpr int PF_KCHUNK = 16;  // key blocks per chunk
+constexpr int PF_MID_MAX = 1024;                                   // longest prompt of the one-workgroup-per-CU builds
+constexpr int PF_MAX_QB = MAX_SEQ_LIMIT / PF_QR;                   // query blocks of the longest prompt
+constexpr int PF_MAX_CHUNKS = MAX_SEQ_LIMIT / (PF_QB * PF_KCHUNK);  // chunks of the longest key range
+constexpr int PF_MAX_PARTS = MAX_SEQ_LIMIT / (PF_QB * PF_KSUB);     // groups of the longest key range
+constexpr int PF_MAX_PSLOTS = PF_MAX_QB * PF_MAX_CHUNKS;           // partial-result slots
+constexpr int PF_MAX_UNITS = PF_MAX_QB * PF_MAX_CHUNKS;            // work units of a kv head
+struct PfPlan {
+  // work units, longest first: query block b | unit c << 6 | (units s of the item - 1) << 9; unit c is
+  // key blocks unit_blocks * c .. (unit_blocks: PF_KCHUNK or PF_KSUB)
+  int nunits, unit_blocks;
+  unsigned short unit[PF_MAX_UNITS];
+  unsigned char pslot[PF_MAX_QB];  // first partial slot of each query block with several units
+};
+struct PfUnit {
+  int b, c, s;
+};
+QL_HD PfUnit pf_unit(unsigned e) { return {(int)(e & 63u), (int)((e >> 6) & 7u), (int)((e >> 9) & 7u) + 1}; }
+QL_HD int pf_key_blocks(int n, int start, int b) {
+  return ((PF_QR * b + PF_QR < n ? PF_QR * b + PF_QR : n) - 1 + start) / PF_QB + 1;
+}
+// The units of `blocks` key blocks each, sorted longest first (ties: later query block first, then key
+// order), the order in which the kernel deals them out. False if they do not fit the tables.
+inline bool pf_plan_units(int n, int start, int blocks, PfPlan& P) {
+  const int nqb = (n + PF_QR - 1) / PF_QR;
+  if (nqb > PF_MAX_QB) return false;
+  struct U {
+    int cost, b, c, s;
+  } u[PF_MAX_UNITS];
+  int nu = 0, slot = 0;
+  for (int b = 0; b < nqb; ++b) {
+    const int nkb = pf_key_blocks(n, start, b), sb = (nkb + blocks - 1) / blocks;
+    if (sb > PF_MAX_PARTS || nu + sb > PF_MAX_UNITS || (sb > 1 && slot + sb > PF_MAX_PSLOTS)) return false;
+    P.pslot[b] = (unsigned char)(sb > 1 ? slot : 0);
+    if (sb > 1) slot += sb;
+    for (int c = 0; c < sb; ++c) u[nu++] = {std::min(blocks, nkb - blocks * c), b, c, sb};
+  }
+  std::sort(u, u + nu, [](const U& x, const U& y) {
+    if (x.cost != y.cost) return x.cost > y.cost;
+    if (x.b != y.b) return x.b > y.b;
+    return x.c < y.c;
+  });
+  for (int i = 0; i < nu; ++i) P.unit[i] = (unsigned short)(u[i].b | u[i].c << 6 | (u[i].s - 1) << 9);
+  P.nunits = nu;
+  P.unit_blocks = blocks;
+  return true;
+}
+// The plan of a call. Units are groups rather than chunks, in the one-workgroup-per-CU builds, where the
+// longest key range is a single group (nothing to merge; 15 positions: 5.4 against 6.4 us per layer) or
+// more than two, and all groups fit one per workgroup: 61 positions after 1400, 11.5 us per layer against
+// 20.8 with chunks; 256 after 500, 10.8 against 15.4. With two rounds of groups the merges cost more than
+// the split gains (256 after 1000: 24.5 against 20.9), and ranges of two groups are as fast as chunks
+// shared by the halves of a workgroup, with nothing to publish (500 positions: 11.6 against 11.4; 400:
+// 11.2 against 10.4).
+inline bool pf_plan(int n, int start, PfPlan& P) {
+  const int nkb = (start + n - 1) / PF_QB + 1;  // of the longest key range
+  if (n <= PF_MID_MAX && (nkb <= PF_KSUB || nkb > 2 * PF_KSUB) && pf_plan_units(n, start, PF_KSUB, P) &&
+      P.nunits * NKV <= NWG)
+    return true;
+  return pf_plan_units(n, start, PF_KCHUNK, P);
+}
 
 // ---- 64-bit values through a 32-bit lane broadcast -----------------------------------
 // `bcast` stands for the GPU's readfirstlane, which takes and returns a signed int. Each

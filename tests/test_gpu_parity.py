@@ -25,6 +25,7 @@ import torch
 
 import qwen_weights as qw
 from oracle import qwen3_oracle as orc
+from test_prefill_plan import PIECES
 
 pytestmark = pytest.mark.gpu
 
@@ -304,12 +305,13 @@ def test_batched_prefill_chunked_equals_whole(ext, full, n, cuts):
     assert torch.equal(a.hidden, b.hidden)
 
 
-@pytest.mark.parametrize("sizes", [(1, 15, 16, 17, 63, 64, 65, 127, 128, 129, 255, 256, 257), (512, 511, 1024), (513, 1023, 511)])
+@pytest.mark.parametrize("sizes", [(1, 15, 16, 17, 63, 64, 65, 127, 128, 129, 255, 256, 257), (512, 511, 1024), (513, 1023, 511),
+                                   *PIECES])
 def test_batched_prefill_builds_agree(ext, full, sizes):
     """Every prefill build (chosen by a call's length: at most 16, 64, 128, 256, 512, 1024 positions,
     and longer) at the edges of its range, against the longest prompts' build, which the oracle
-    checks: a prompt prefilled in pieces of these sizes leaves the K/V cache and the hidden state of
-    one prefill of all of it, bit for bit. Run twice: the second pass finds the buffers of the first."""
+    checks: a prompt prefilled in pieces of these sizes (PIECES: later turns, whose attention merges 1 to 8
+    groups of keys) leaves the K/V cache and the hidden state of one prefill of all of it, bit for bit. Run twice: the second pass finds the buffers of the first."""
     hw, w, packed = full
     n = sum(sizes)
     assert n > 1024
