@@ -177,7 +177,7 @@ constexpr bool kTrace = false;
 constexpr bool kSample = false;
 constexpr bool kTopK = false;
 constexpr bool kDist = false;
-constexpr bool kOwnLayer = false;
+constexpr bool kMlp = false;
 #include "decode_body.inc"
 }  // namespace fast
 
@@ -186,7 +186,7 @@ constexpr bool kTrace = true;
 constexpr bool kSample = false;
 constexpr bool kTopK = false;
 constexpr bool kDist = false;
-constexpr bool kOwnLayer = false;
+constexpr bool kMlp = false;
 #include "decode_body.inc"
 }  // namespace traced
 
@@ -195,7 +195,7 @@ constexpr bool kTrace = false;
 constexpr bool kSample = true;
 constexpr bool kTopK = true;
 constexpr bool kDist = false;
-constexpr bool kOwnLayer = false;
+constexpr bool kMlp = false;
 #include "decode_body.inc"
 }  // namespace sampled
 
@@ -206,7 +206,7 @@ constexpr bool kTrace = false;
 constexpr bool kSample = true;
 constexpr bool kTopK = true;
 constexpr bool kDist = true;
-constexpr bool kOwnLayer = false;
+constexpr bool kMlp = false;
 #include "decode_body.inc"
 }  // namespace dsampled
 
@@ -217,19 +217,19 @@ constexpr bool kTrace = false;
 constexpr bool kSample = true;
 constexpr bool kTopK = false;
 constexpr bool kDist = false;
-constexpr bool kOwnLayer = false;
+constexpr bool kMlp = false;
 #include "decode_body.inc"
 }  // namespace tsampled
 
-// the isolated MLP block: the greedy build with the one layer's pointers in the arguments (a table in
-// memory took a copy that the host waited for, or a kernel of its own: 15.9 -> 11.1 us per call; the
-// same choice at run time in the greedy build made its tokens 1% slower, by its scalar registers)
+// the isolated MLP block alone, with the one layer's pointers in the arguments (a table in memory took a
+// copy that the host waited for, or a kernel of its own: 15.9 -> 11.1 us per call; the same choice at run
+// time in the greedy build made its tokens 1% slower, by its scalar registers)
 namespace isolated {
 constexpr bool kTrace = false;
 constexpr bool kSample = false;
 constexpr bool kTopK = false;
 constexpr bool kDist = false;
-constexpr bool kOwnLayer = true;
+constexpr bool kMlp = true;
 #include "decode_body.inc"
 }  // namespace isolated
 
