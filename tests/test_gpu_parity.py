@@ -18,6 +18,7 @@ qwen_megakernel_C -> libqwen_megakernel.so (or the C-ABI directly via ctypes).
 import ctypes
 import math
 import os
+import threading
 
 import numpy as np
 import pytest
@@ -363,6 +364,49 @@ def test_calls_on_two_streams_in_turn(ext, full):
         assert ext.last_error() == 0
         for g in got:
             assert all(torch.equal(p, q) for p, q in zip(g, want))
+
+
+def test_calls_from_two_threads(ext, full):
+    """Two threads, each with a stream and buffers of its own, make calls at the same time: each gets what
+    it gets alone (the calls share the device's workspaces and take turns)."""
+    hw, w, packed = full
+    prompts = [torch.tensor(qw.synthetic_prompt(n, seed=66 + n), dtype=torch.int32, device="cuda") for n in (20, 150)]
+
+    def calls(k, run, lo):
+        n = prompts[k].numel()
+        ext.prefill(prompts[k], w["embed_weight"], packed, w["cos_table"], w["sin_table"], run.kc, run.vc, run.hidden, 2,
+                    0, MAX_SEQ, SCALE)
+        toks = ext.generate_ex(5 + k, 3, None, w["embed_weight"], packed, w["final_norm_weight"], w["lm_head_weight"],
+                               w["cos_table"], w["sin_table"], run.kc, run.vc, run.hidden, run.norm_out, lo, None, 2, n,
+                               MAX_SEQ, SCALE)
+        return [run.kc, run.vc, lo, toks, ext.sample(lo[0], 0.8, 0, 0.9, 3, 7)]
+
+    runs = [Run(w, packed, 2) for _ in range(2)]
+    los = [torch.empty(3, V, dtype=torch.float32, device="cuda") for _ in range(2)]
+    want = [[x.clone() for x in calls(k, runs[k], los[k])] for k in range(2)]
+    torch.cuda.synchronize()
+    bad = []
+
+    def worker(k):
+        try:
+            stream = torch.cuda.Stream()
+            with torch.cuda.stream(stream):
+                for _ in range(20):
+                    got = calls(k, runs[k], los[k])
+                    stream.synchronize()
+                    if not all(torch.equal(p, q) for p, q in zip(got, want[k])):
+                        bad.append(k)
+        except Exception as e:  # a thread's failure has to reach the test
+            bad.append(e)
+
+    threads = [threading.Thread(target=worker, args=(k,)) for k in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert not bad, bad
+    assert ext.last_error() == 0
 
 
 def test_replayed_prefill_beside_eager_calls(ext, full):
