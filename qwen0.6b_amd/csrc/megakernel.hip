@@ -294,8 +294,7 @@ struct DeviceState {
 
 std::mutex g_mu;
 DeviceState g_dev[MAX_DEVICES];
-// What the library allocates (workspaces, the prefill and
-// sampler buffers) is held until the process ends and released with it; no exit handler
+// What the library allocates (workspaces, the prefill and sampler buffers) is held until the process ends and released with it; no exit handler
 // calls into the HIP runtime.
 
 int zero_words(void* p, long bytes, hipStream_t s) {
@@ -306,7 +305,7 @@ int zero_words(void* p, long bytes, hipStream_t s) {
 // The prefill builds: one-workgroup-per-CU kernels with tiles for at most 16, 64, .. 1024 positions, then
 // the two-workgroups-per-CU kernel for longer prompts. The last line lies where 128-position tiles stop
 // giving one tile per CU (1025 positions are 288 QKV tiles for 256 workgroups): at 999 positions the
-// short build takes 2.35 ms against 2.85, at 1919 a one-workgroup-per-CU build 3.83 against 3.72.
+// short build takes 2.41 ms against 2.86, at 1919 a one-workgroup-per-CU build 3.83 against 3.72.
 constexpr int PF_CLASS_MAX[] = {16, 64, 128, 256, 512, 1024};
 constexpr int PF_CLASSES = sizeof(PF_CLASS_MAX) / sizeof(int);
 static_assert(PF_CLASS_MAX[PF_CLASSES - 1] == PF_MID_MAX, "class limits");
@@ -351,9 +350,9 @@ static_assert(sizeof(BUILDS) / sizeof(Build) == PREFILL + PF_CLASSES + 1, "a bui
 // its own, 18-20 us per call (a sampler launch with nothing to select 27 -> 7 us, the lm_head 78 ->
 // 63); an event recorded after a plain launch costs 3 us more than one that belongs to it.
 // A captured call puts the same wait and the same record into the graph, as event nodes, so that each
-// replay waits for the launch before it and later ones wait for the replay (the order is that of the
-// host's calls, hipGraphLaunch among them). Its launch is a cooperative one: replays that several
-// threads launch at once are then still taken one after the other.
+// replay waits for the launch before it and later ones wait for the replay: the order is that of the
+// host's calls, hipGraphLaunch among them, which the program makes one after the other. (Its launch stays
+// a cooperative one: grids of replays that threads launch at once, out of any order, do not meet.)
 
 // Whether the stream is being captured. Where the runtime cannot say (or the capture has failed) nothing
 // may be sent to the stream: a launch taken for a captured one would be in no order.
