@@ -144,8 +144,8 @@ int qwen_generate_until(
  * kernel, never hipMemset. Not for stream capture: on a stream that is being
  * captured it returns QWEN_ERR_ARG (the exchange tags' token epochs are launch
  * arguments, so a replayed graph would reuse them). Every call on a GPU shares
- * that GPU's array: calls that overlap on one GPU (two streams, two threads)
- * race and must be serialized by the caller. Errors are reported by
+ * that GPU's array: like all of the library's launches on a GPU they follow
+ * each other, whatever their streams and threads. Errors are reported by
  * qwen_last_error(). */
 int qwen_generate_nosync_noalloc(
     int first_token_id, int num_steps, const void* embed_weight,
